@@ -363,3 +363,40 @@ def test_two_stage_groups(torch, ctx, m, k, n):
     print(f"two stage groups q8 {m}x{k}x{n}: max abs {err:.2e} (bar {bar:.1e})", flush=True)
     assert np.all(np.isfinite(outs[0])) and err <= bar
     assert np.array_equal(outs[0], outs[1])
+
+
+# One case per branch of the packed kernels' dispatch, at the edges of their tiles: one chunk of k per
+# workgroup (k split, 64-column tiles), several (128 or 256 columns), unsplit calls with fewer and more
+# 128-column units than CUs; one and two m-tiles and 64-row blocks with a ragged last one; n not a
+# multiple of 4 (4-byte stores), of 32 or of a tile; stage counts odd, even and past three.
+PACKED_CASES = [(1, 512, 70), (32, 288, 33), (31, 8960, 130), (33, 768, 257), (64, 8960, 1536), (129, 4864, 897),
+                (200, 1280, 4100), (48, 1376, 16386), (64, 544, 40004), (7, 480, 9001), (256, 96, 8200)]
+
+
+@pytest.mark.parametrize("epilogue", ["none", "gelu", "add"])
+@pytest.mark.parametrize("m,k,n", PACKED_CASES)
+def test_packed_dispatch_branches(torch, ctx, m, k, n, epilogue):
+    """Against f64 over the dequantized weights (bar as above: 2e-5 sqrt(k) on outputs of unit scale; GELU's
+    slope is below 1.13), the rows past m untouched."""
+    from zwhisper_amd import _lib
+
+    x, w, b = inputs(m + 3 * k + 5 * n, m, k, n)
+    xd, bd = torch.from_numpy(x).cuda(), torch.from_numpy(b).cuda()
+    ref = ref64(x, w, b)
+    rng = np.random.default_rng(m * n)
+    old = rng.standard_normal((m + 1, n)).astype(np.float32)
+    if epilogue == "gelu":
+        ref = 0.5 * ref * (1.0 + np.tanh(0.7978845608028654 * (ref + 0.044715 * ref ** 3)))
+    elif epilogue == "add":
+        ref = ref + old[:m]
+    out = torch.from_numpy(old).cuda()
+    epi = {"none": _lib.EPI_NONE, "gelu": _lib.EPI_GELU, "add": _lib.EPI_ADD}[epilogue]
+    with w.resident(ctx) as rw:
+        ctx.linear_q8w_epi_dev(xd, m, rw, bd, out, epi)
+        torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    err = float(np.abs(got[:m] - ref).max())
+    bar = 1.13 * 2e-5 * np.sqrt(k)
+    print(f"packed q8 {m}x{k}x{n} {epilogue}: max abs {err:.2e} (bar {bar:.1e})", flush=True)
+    assert np.all(np.isfinite(got)) and err <= bar
+    assert np.array_equal(got[m], old[m])

@@ -144,6 +144,8 @@ std::string check_linear(uint64_t m, uint64_t k, uint32_t w_type, uint64_t n) {
 #define ZWG_Q8P_SPLIT_TARGET 256
 #endif
 template <int MT>
+hipError_t launch_xprep(const float *x, _Float16 *xcvt, int32_t m, int32_t k, int32_t n_chunks, hipStream_t stream);
+template <int MT>
 int run_q8_stream_mt(zwg_ctx *ctx, const zwg_lin::Q8Args &base) {
     zwg_lin::Q8Args a = base;
     const uint64_t m = (uint64_t)a.m, n = (uint64_t)a.n;
@@ -163,11 +165,7 @@ int run_q8_stream_mt(zwg_ctx *ctx, const zwg_lin::Q8Args &base) {
     _Float16 *xcvt = reinterpret_cast<_Float16 *>(ctx->workspace);
     a.part = n_split > 1 ? reinterpret_cast<float *>(reinterpret_cast<char *>(ctx->workspace) + part_off) : nullptr;
 
-    const int64_t prep_threads = (int64_t)n_chunks * MT * 32 * (zwg_lin::kQ8Chunk / 4);
-    const int prep_bs = small_block(prep_threads);
-    zwg_lin::linear_q8_xprep_kernel<MT><<<blocks_for(prep_threads, prep_bs), prep_bs, 0, ctx->stream>>>(
-        a.x, xcvt, a.m, a.k, n_chunks);
-    hipError_t e = hipGetLastError();
+    hipError_t e = launch_xprep<MT>(a.x, xcvt, a.m, a.k, n_chunks, ctx->stream);
     if (e != hipSuccess) return fail_hip(ctx, "linear (int8) x preparation launch", e);
     dim3 grid((unsigned)gx, (unsigned)n_split);
     if (S == 2) zwg_lin::linear_q8_stream_kernel<MT, 2><<<grid, zwg_lin::kQ8Threads, 0, ctx->stream>>>(a, xcvt);
@@ -182,45 +180,28 @@ int run_q8_stream_mt(zwg_ctx *ctx, const zwg_lin::Q8Args &base) {
     return ZWG_OK;
 }
 
-// Resident packed weights with m <= 64, one or more weight sets over the same x (g.count sets;
-// q/scales/n_slabs/n/bias/out filled by the caller): one stream launch over every set's
-// workgroups (four slabs of 32 rows each), preceded by one x split for 64-row calls (32-row calls
-// split x inside the stream kernel), and when k is split, one split sum over every set's outputs.
-// The k split is chosen from the group's total workgroup count, as for a single call: a call of
-// fewer than ZWG_Q8P_SPLIT_BELOW workgroups is split until it has about 512.
-#ifndef ZWG_Q8P_WAVES
-#define ZWG_Q8P_WAVES 4
-#endif
-#ifndef ZWG_Q8P_WAVES_32
-#define ZWG_Q8P_WAVES_32 2
-#endif
-// waves (one 32-row slab each) sharing each x stage of the packed stream kernel: four for 64-row
-// calls (8 measured 5-9% slower on the logits and decode-step workloads: half the workgroups,
-// longer tails; 2 measured 4% slower on the Qwen2.5-1.5B step and 26% on its logits), two for
-// 32-row calls, whose x stage is half as large (Whisper small.en step 675 -> 651 us against 4)
+// Resident packed weights, one or more weight sets over the same x (g.count sets;
+// q/scales/n_slabs/n/bias/out filled by the caller): one launch over every set's workgroups,
+// preceded by one x split for the 64-row calls that do not split x themselves, and when k is split,
+// one split sum over every set's outputs.  The k split is chosen from the group's total count of
+// units of q8p_unit<MT>() weight rows, as for a single call; the kernel and its tile are chosen
+// below from the split and the unit count, and do not change the sums.
 template <int MT>
-constexpr int q8p_waves() { return MT == 1 ? ZWG_Q8P_WAVES_32 : ZWG_Q8P_WAVES; }
+constexpr int q8p_unit() { return MT == 1 ? 64 : 128; }
 // k is split only for calls below this many workgroups.  A call at or above it streams unsplit:
 // its partial sums would be as large as half its weights (the Qwen2.5-1.5B gate/up, 140
 // workgroups: split 3 ways, 13.8 MB of partials for 27.5 MB of weights).  Measured on one box,
 // splitting below 512 / 160 / 100 / 64 workgroups: Qwen2.5-1.5B decode step 2297 / 2297 / 2126 /
 // 2118 us, small.en decoder step 690 / 675 / 675 / 675 us.
-#ifndef ZWG_Q8P_XS_SPLIT
-#define ZWG_Q8P_XS_SPLIT 1
-#endif
 #ifndef ZWG_Q8P_SPLIT_BELOW
 #define ZWG_Q8P_SPLIT_BELOW 128
-#endif
-// unsplit calls of fewer workgroups than this run two stage groups per workgroup (each over half
-// of k, summed through LDS at the end)
-#ifndef ZWG_Q8P_KS_BELOW
-#define ZWG_Q8P_KS_BELOW 256
 #endif
 // calls of up to this many rows stream the resident weights (64-row blocks of one launch); more
 // rows take the tiled GEMM
 #ifndef ZWG_Q8P_STREAM_ROWS
 #define ZWG_Q8P_STREAM_ROWS 256
 #endif
+#define ZWG_Q8P_FUSED_ROWS 256
 
 
 // Row kernels of n <= 2048 floats (a wave per row, n / 256 float4 per lane, rounded up), one
@@ -308,13 +289,83 @@ bool q8p_split_k(int64_t gx, int n_chunks, int nz = 1) {
 // own first.
 template <int MT>
 bool q8p_splits_x_itself(int64_t gx, int n_chunks) {
-    return MT == 1 || (ZWG_Q8P_XS_SPLIT && q8p_split_k(gx, n_chunks));
+    return MT == 1 || q8p_split_k(gx, n_chunks);
 }
+// x split into f16 hi/lo halves for every 32 MT-row block, into xcvt
+template <int MT>
+hipError_t launch_xprep(const float *x, _Float16 *xcvt, int32_t m, int32_t k, int32_t n_chunks, hipStream_t stream) {
+    const int64_t nz = (m + 32 * MT - 1) / (32 * MT);
+    const int64_t threads = nz * n_chunks * MT * 32 * (zwg_lin::kQ8Chunk / 4);
+    const int bs = small_block(threads);
+    zwg_lin::linear_q8_xprep_kernel<MT><<<blocks_for(threads, bs), bs, 0, stream>>>(x, xcvt, m, k, n_chunks);
+    return hipGetLastError();
+}
+
+// One launch of a packed-weight kernel over tiles of 32 MT rows x 32 NS columns; NS x G waves, G
+// along the m-tiles (SHORT) or the blocks of a stage
+template <bool SHORT, int MT, int NS, int G, int SB>
+hipError_t launch_q8p_tile(const zwg_lin::Q8Args &a, zwg_lin::Q8Group g, const _Float16 *xcvt, bool XS, int n_split, int nz,
+                           hipStream_t stream) {
+    using namespace zwg_lin;
+    const bool pair = g.swiglu != 0;
+    int64_t gx = 0; // a SwiGLU pair's workgroups each take half their columns from both sets
+    for (int j = 0; j < kQ8MaxGroup; ++j) {
+        g.block_start[j] = (int32_t)gx;
+        if (j < (pair ? 1 : g.count)) gx += ((int64_t)g.n[j] + (pair ? 16 : 32) * NS - 1) / ((pair ? 16 : 32) * NS);
+    }
+    g.block_start[kQ8MaxGroup] = (int32_t)gx;
+    const dim3 grid((unsigned)gx, (unsigned)n_split, (unsigned)nz);
+    const auto go = [&](auto xs, auto pr, auto gr) {
+        if constexpr (SHORT)
+            linear_q8p_short_kernel<MT, NS, G, decltype(xs)::value, decltype(pr)::value, decltype(gr)::value>
+                <<<grid, 64 * NS * G, 0, stream>>>(a, g, xcvt);
+        else
+            linear_q8p_long_kernel<MT, NS, G, SB, decltype(xs)::value, decltype(pr)::value, decltype(gr)::value>
+                <<<grid, 64 * NS * G, 0, stream>>>(a, g, xcvt);
+    };
+    const auto with_form = [&](auto xs) {
+        if (pair) go(xs, std::true_type{}, std::true_type{});
+        else if (g.count > 1) go(xs, std::false_type{}, std::true_type{});
+        else go(xs, std::false_type{}, std::false_type{});
+    };
+    if constexpr (MT == 1) with_form(std::true_type{}); // 32-row calls always split x themselves
+    else if (XS) with_form(std::true_type{});
+    else with_form(std::false_type{});
+    return hipGetLastError();
+}
+
+// The kernel and tile of a call of `units` q8p_unit<MT>() x 32 MT-row units, n_split ways, nz row
+// blocks; the lines are where the measured times cross (back to back, weights from HBM, us).
+template <int MT>
+hipError_t launch_q8p(const zwg_lin::Q8Args &a, const zwg_lin::Q8Group &g, const _Float16 *xcvt, bool XS, int64_t units,
+                      int n_split, int nz, hipStream_t st) {
+    if constexpr (MT == 1) {
+        // one chunk per workgroup: 64 columns (32 x 768 x 768 in 3 splits 4.7, 128 columns 4.9); two or
+        // more: 128 columns, half the x reads (32 x 8960 x 1536 in 18 splits 8.2, 64 columns 11.2)
+        if (n_split > 1 && a.chunks_per_split == 1) return launch_q8p_tile<true, 1, 2, 1, 4>(a, g, xcvt, XS, n_split, nz, st);
+        if (n_split > 1) return launch_q8p_tile<true, 1, 4, 1, 4>(a, g, xcvt, XS, n_split, nz, st);
+        // unsplit: 1 x 896 x 151936 31 (64 columns 42, 256 columns 38), 32 x 768 x 51864 16.0 (19, 15.4)
+        return launch_q8p_tile<false, 1, 4, 1, 4>(a, g, xcvt, XS, n_split, nz, st);
+    } else {
+        // one chunk per workgroup: 64 columns on four waves (64 x 1536 x 1536 in 6 splits 5.7, 128
+        // columns 6.6, the long kernel 6.9)
+        if (n_split > 1 && a.chunks_per_split == 1) return launch_q8p_tile<true, 2, 2, 2, 4>(a, g, xcvt, XS, n_split, nz, st);
+        // more units than CUs, split: 256 columns (256 x 4864 x 896 in 10 splits 14.5, 128 columns
+        // 16.1); fewer: 128 columns (64 x 8960 x 1536 in 18 splits 12.0, 256 columns 13.9)
+        if (n_split > 1 && units * n_split > 256) return launch_q8p_tile<false, 2, 8, 1, 2>(a, g, xcvt, XS, n_split, nz, st);
+        // unsplit with fewer units than CUs: two waves per SIMD, each on half of every stage's blocks (a
+        // 64-row SwiGLU pair of 8960 x 1536, 140 units: four waves 22.7)
+        if (n_split == 1 && units < 256) return launch_q8p_tile<false, 2, 4, 2, 4>(a, g, xcvt, XS, n_split, nz, st);
+        // 64 x 1536 x 151936 79 (256 columns 90), 1001 x 1536 x 8960 73 (86)
+        return launch_q8p_tile<false, 2, 4, 1, 2>(a, g, xcvt, XS, n_split, nz, st);
+    }
+}
+
 template <int MT>
 int run_q8p_group(zwg_ctx *ctx, const zwg_lin::Q8Args &base, zwg_lin::Q8Group g,
                   const zwg_lin::Q8KvStore *kvs = nullptr, const zwg_lin::Q8ResLn *resln = nullptr,
                   Q8PartsOut *po = nullptr, const _Float16 *xcvt_in = nullptr) {
-    constexpr int kQ8pWaves = q8p_waves<MT>();
+    constexpr int kUnit = q8p_unit<MT>();
     zwg_lin::Q8Args a = base;
     const uint64_t m = (uint64_t)a.m;
     const bool pair = g.swiglu != 0;
@@ -323,35 +374,29 @@ int run_q8p_group(zwg_ctx *ctx, const zwg_lin::Q8Args &base, zwg_lin::Q8Group g,
     int64_t gx = 0;
     uint64_t n_tot = 0;
     for (int j = 0; j < zwg_lin::kQ8MaxGroup; ++j) {
-        g.block_start[j] = (int32_t)gx;
         g.elem_start[j] = (int64_t)(m * n_tot);
         if (j < g.count) {
-            gx += (g.n[j] + 32 * kQ8pWaves - 1) / (32 * kQ8pWaves);
+            gx += (g.n[j] + kUnit - 1) / kUnit;
             n_tot += (uint64_t)g.n[j];
         }
     }
-    g.block_start[zwg_lin::kQ8MaxGroup] = (int32_t)gx;
     g.elem_start[zwg_lin::kQ8MaxGroup] = (int64_t)(m * n_tot);
     const int n_chunks = (a.k + zwg_lin::kQ8Chunk - 1) / zwg_lin::kQ8Chunk;
     g.n_chunks = n_chunks;
-    // a SwiGLU pair's workgroups each take the same columns of both sets: the grid covers one
-    // set's columns at half the rows per workgroup, while every choice below is the two sets'
-    // unpaired one (so the sums are the same as the pair's two separate outputs')
-    const int64_t gx_launch = pair ? ((int64_t)g.n[0] + 16 * kQ8pWaves - 1) / (16 * kQ8pWaves) : gx;
-    // calls of more than 64 rows: nz blocks of 64 rows in one launch (gridDim.z), x split in the
-    // kernel, and the k split chosen from all nz gx workgroups
+    // calls of more than 64 rows: nz blocks of 64 rows in one launch (gridDim.z), and the k split
+    // chosen from all nz gx units
     const int nz = (int)((m + 32 * MT - 1) / (32 * MT));
-    if (nz > 1 && (MT != 2 || po || xcvt_in || (resln && resln->xcvt)))
-        return fail(ctx, "the split rows and partials calls take at most 64 rows");
+    if (nz > 1 && (MT != 2 || po)) return fail(ctx, "the partials call takes at most 64 rows");
     const int64_t gxz = gx * nz;
-    const bool split_k = q8p_split_k(gxz, n_chunks, nz);
-    // xcvt_in (a 64-row call): x was split by the caller's previous launch.  The partial sums keep
-    // the place (and so the split count) the call has without it.
-    const bool xs_own = q8p_splits_x_itself<MT>(gxz, n_chunks) || nz > 1;
+    const bool split_k = q8p_split_k(gxz, n_chunks, nz) && m <= ZWG_Q8P_FUSED_ROWS;
+    // xcvt_in (64-row blocks): x was split by the caller's previous launch.  The partial sums keep
+    // the place (and so the split count) the call has without it.  Calls of at most 256 rows whose
+    // row blocks share one launch split x themselves; longer ones (always unsplit) take the pass.
+    const bool long_m = m > ZWG_Q8P_FUSED_ROWS;
+    const bool xs_own = q8p_splits_x_itself<MT>(gxz, n_chunks) || (nz > 1 && !long_m);
     const bool XS = xs_own && !(MT == 2 && xcvt_in);
-    if (resln && resln->xcvt && (ZWG_ADDLN_WIDE == 0 || MT != 2))
-        return fail(ctx, "split rows for the next call come from 33..64-row calls' one-thread-per-column sums");
-    const uint64_t xcvt_bytes = xs_own ? 0 : (uint64_t)n_chunks * zwg_lin::q8_chunk_halves<MT>() * 2;
+    if (resln && resln->xcvt && MT != 2) return fail(ctx, "split rows for the next call come from calls of more than 32 rows");
+    const uint64_t xcvt_bytes = xs_own ? 0 : (uint64_t)nz * n_chunks * zwg_lin::q8_chunk_halves<MT>() * 2;
     const uint64_t part_off = (xcvt_bytes + 255) / 256 * 256;
     if (part_off > ctx->workspace_bytes) return fail(ctx, "workspace too small for this linear call");
     int n_split = 1;
@@ -381,34 +426,10 @@ int run_q8p_group(zwg_ctx *ctx, const zwg_lin::Q8Args &base, zwg_lin::Q8Group g,
     const _Float16 *xcvt = XS ? nullptr : xcvt_in ? xcvt_in : reinterpret_cast<_Float16 *>(ctx->workspace);
     hipError_t e;
     if (!XS && !xcvt_in) {
-        const int64_t prep_threads = (int64_t)n_chunks * MT * 32 * (zwg_lin::kQ8Chunk / 4);
-        const int prep_bs = small_block(prep_threads);
-        zwg_lin::linear_q8_xprep_kernel<MT><<<blocks_for(prep_threads, prep_bs), prep_bs, 0, ctx->stream>>>(
-            a.x, reinterpret_cast<_Float16 *>(ctx->workspace), a.m, a.k, n_chunks);
-        e = hipGetLastError();
+        e = launch_xprep<MT>(a.x, reinterpret_cast<_Float16 *>(ctx->workspace), a.m, a.k, n_chunks, ctx->stream);
         if (e != hipSuccess) return fail_hip(ctx, "linear (int8) x preparation launch", e);
     }
-    dim3 grid((unsigned)gx_launch, (unsigned)n_split, (unsigned)nz);
-    // unsplit calls of too few workgroups to fill the chip: two stage groups per workgroup
-    const bool two_groups = n_split == 1 && gxz < ZWG_Q8P_KS_BELOW && n_chunks > 1;
-    using namespace zwg_lin;
-    constexpr int W = kQ8pWaves;
-    if (pair) {
-        if (two_groups) {
-            if (XS) linear_q8p_stream_kernel<MT, 1, W, true, 2, true><<<grid, 128 * W, 0, ctx->stream>>>(a, g, xcvt);
-            else linear_q8p_stream_kernel<MT, 1, W, false, 2, true><<<grid, 128 * W, 0, ctx->stream>>>(a, g, xcvt);
-        } else {
-            if (XS) linear_q8p_stream_kernel<MT, 1, W, true, 1, true><<<grid, 64 * W, 0, ctx->stream>>>(a, g, xcvt);
-            else linear_q8p_stream_kernel<MT, 1, W, false, 1, true><<<grid, 64 * W, 0, ctx->stream>>>(a, g, xcvt);
-        }
-    } else if (two_groups) {
-        if (XS) linear_q8p_stream_kernel<MT, 1, W, true, 2><<<grid, 128 * W, 0, ctx->stream>>>(a, g, xcvt);
-        else linear_q8p_stream_kernel<MT, 1, W, false, 2><<<grid, 128 * W, 0, ctx->stream>>>(a, g, xcvt);
-    } else {
-        if (XS) linear_q8p_stream_kernel<MT, 1, W, true><<<grid, 64 * W, 0, ctx->stream>>>(a, g, xcvt);
-        else linear_q8p_stream_kernel<MT, 1, W, false><<<grid, 64 * W, 0, ctx->stream>>>(a, g, xcvt);
-    }
-    e = hipGetLastError();
+    e = launch_q8p<MT>(a, g, xcvt, XS, gxz, n_split, nz, ctx->stream);
     if (e != hipSuccess) return fail_hip(ctx, "linear (int8 stream) kernel launch", e);
     if (kvs) {
         const int64_t threads = (int64_t)m * (kvs->n_head + 2 * kvs->n_head_kv) * (kvs->d / 8);
@@ -746,7 +767,7 @@ int zwg_host::linear_q8w_add_ln(zwg_ctx *ctx, const float *xin, uint64_t m, cons
 
 bool zwg_host::q8w_group_reads_xcvt(uint64_t m, uint32_t n_w, const zwg_q8w *const *w) {
     if (m <= 32 || m > 64 || n_w == 0 || n_w > (uint32_t)zwg_lin::kQ8MaxGroup) return false;
-    constexpr int kRows = 32 * q8p_waves<2>();
+    constexpr int kRows = q8p_unit<2>();
     int64_t gx = 0;
     for (uint32_t j = 0; j < n_w; ++j) gx += ((int64_t)w[j]->n + kRows - 1) / kRows;
     const int n_chunks = (int)((w[0]->k + zwg_lin::kQ8Chunk - 1) / zwg_lin::kQ8Chunk);

@@ -39,6 +39,7 @@
 #include <stdint.h>
 
 #include "elementwise.hpp"
+#include "f16_split.hpp"
 #include "kv_image.hpp"
 
 namespace zwg_lin {

@@ -75,14 +75,16 @@ struct Q8Args {
 
 // Layout of x's hi/lo halves, per chunk of 256 k: [block][m-tile][hi/lo][k-step][lane][8 halves],
 // 32 KB per m-tile.  Lane l, k-step s of (block b, m-tile i) holds x[32 i + l % 32][kb + 16 (l / 32)
-// + 8 s + 0..7], kb = 32 b.  One [hi/lo][k-step] piece of a (block, m-tile) is 1 KB: 64 lanes x 16 B.
+// + 8 s + 0..7], kb = 32 b.  One [hi/lo][k-step] piece of a (block, m-tile) is 1 KB: 64 lanes x 16 B,
+// lane l at place l ^ 4 s: a write of four consecutive k of each row touches both k-steps, which
+// then sit on different banks.
 template <int MT>
 __host__ __device__ constexpr int q8_chunk_halves() {
     return kQ8ChunkBlocks * MT * 2 * 2 * 64 * 8;
 }
 template <int MT>
 __device__ __forceinline__ int q8_xs_at(int b, int i, int hl, int s, int lane) {
-    return ((((b * MT + i) * 2 + hl) * 2 + s) * 64 + lane) * 8;
+    return ((((b * MT + i) * 2 + hl) * 2 + s) * 64 + (lane ^ (4 * s))) * 8;
 }
 
 // x[row][gk .. gk + 3] (gk % 4 == 0) split into f16 hi/lo halves at its place in xcvt's chunk
@@ -94,30 +96,28 @@ __device__ __forceinline__ void q8_xs_store(_Float16 *xcvt, int row, int gk, f32
     const int gg = kb >> 4, s = (kb >> 3) & 1, j = kb & 7;
     const int i = row >> 5, l = (row & 31) + 32 * gg;
     half4 hi, lo;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-        hi[e] = (_Float16)v[e];
-        lo[e] = (_Float16)(v[e] - (float)hi[e]);
-    }
+    zwg_split::split4(v, hi, lo);
     _Float16 *base = xcvt + (int64_t)c * q8_chunk_halves<MT>();
     *reinterpret_cast<half4 *>(base + q8_xs_at<MT>(b, i, 0, s, l) + j) = hi;
     *reinterpret_cast<half4 *>(base + q8_xs_at<MT>(b, i, 1, s, l) + j) = lo;
 }
 
-// x f32 [m][k] -> xcvt f16 [n_chunks][chunk layout above]; rows >= m and columns >= k are 0.
-// One thread per 4 consecutive k of one row.
+// x f32 [m][k] -> xcvt f16 [blocks of 32 MT rows][n_chunks][chunk layout above]; rows >= m and columns
+// >= k are 0.  One thread per 4 consecutive k of one row.
 template <int MT>
 __global__ __launch_bounds__(256) void linear_q8_xprep_kernel(const float *x, _Float16 *xcvt, int32_t m, int32_t k,
                                                              int32_t n_chunks) {
     const int64_t f = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const int64_t per_chunk = MT * 32 * (kQ8Chunk / 4);
-    if (f >= per_chunk * n_chunks) return;
-    const int c = (int)(f / per_chunk), rem = (int)(f % per_chunk);
-    const int row = rem / (kQ8Chunk / 4), kk = 4 * (rem % (kQ8Chunk / 4));
-    const int gk = c * kQ8Chunk + kk;
+    const int per_chunk = MT * 32 * (kQ8Chunk / 4);
+    const int64_t zc = f / per_chunk; // row block z, chunk c
+    const int rem = (int)(f % per_chunk);
+    const int z = (int)(zc / n_chunks), c = (int)(zc % n_chunks);
+    const int row = rem / (kQ8Chunk / 4), gk = c * kQ8Chunk + 4 * (rem % (kQ8Chunk / 4));
+    const int64_t r = (int64_t)z * MT * 32 + row;
+    if (z * MT * 32 >= m) return;
     f32x4 v = {0.f, 0.f, 0.f, 0.f};
-    if (row < m && gk < k) v = *reinterpret_cast<const f32x4 *>(x + (int64_t)row * k + gk);
-    q8_xs_store<MT>(xcvt, row, gk, v);
+    if (r < m && gk < k) v = *reinterpret_cast<const f32x4 *>(x + r * k + gk);
+    q8_xs_store<MT>(xcvt + (int64_t)z * n_chunks * q8_chunk_halves<MT>(), row, gk, v);
 }
 
 template <int MT, int S>
@@ -334,310 +334,501 @@ __global__ __launch_bounds__(256) void linear_q8_pack_kernel(const int8_t *q, co
     }
 }
 
-// The stream kernel over packed weights, software-pipelined.  k is walked in stages of 4 blocks
-// (128 k).  x stages sit in LDS double-buffered and each wave keeps two register sets of weights
-// and scales, so the loads of stage t + 1 (x, then weights, then scales) are in flight while stage
-// t's MFMAs run: at the top of stage t the wave waits only for its x of stage t (loads complete in
-// order, and stage t's weights were issued after them), and the barrier that follows tells every
-// wave that the stage's x is in LDS (and that stage t - 1's buffer is free again).  Two x paths:
-//   XS = false: x was split into f16 hi/lo halves in the MFMA A-operand order (q8_xs_at) by
-//     linear_q8_xprep_kernel; each stage's pieces are copied into LDS by direct global-to-LDS loads
-//     (no VGPRs, no VALU).
-//   XS = true: no separate pass.  A stage's f32 x rows arrive in registers (coalesced 16-byte
-//     loads) and each workgroup splits them and writes them into the LDS stage itself before the
-//     barrier.  This costs registers and a short split before each barrier, and saves a launch:
-//     the better trade for 32-row calls and for small 64-row calls whose k is split (measured:
-//     Whisper small.en decoder step 784 -> 681 us, Qwen2.5-1.5B decode step 2095 -> 1960 us), the
-//     worse one for a large unsplit 64-row call (Qwen2.5-1.5B logits 109 -> 150 us).
+// The packed-weight kernels: a workgroup of NS x MS x KB waves computes 32 MT rows x 32 NS columns
+// (weight rows); wave (ws, ms, kg) takes slab ws, m-tiles ms MT / MS .. of it and blocks
+// kg SB / KB .. of every stage.  k is walked in stages of SB blocks.  x stages sit in LDS in the MFMA
+// A-operand order (q8_xs_at) and are shared by the waves; a wave's weights and scales go to its own
+// registers.  Each block's sum starts from zero (four MFMAs) and is scaled into the accumulator in
+// block order, so every tile shape with KB = 1 gives the same bits; with KB = 2 the two waves' sums
+// are added at the end.
+//
+// Loads run ahead of their use.  Past the last stage the same loads go out with out-of-range
+// offsets: they return zeros without touching memory, and every path through a loop then has the
+// same loads in flight, so the compiler's in-order wait counts stay exact.  Two x paths:
+//   XS = false: x was split into f16 hi/lo halves in the MFMA A-operand order by
+//     linear_q8_xprep_kernel (or the previous call's row kernel); each stage's pieces are copied into
+//     LDS by direct global-to-LDS loads (no VGPRs, no VALU).
+//   XS = true: no separate pass.  A stage's f32 x rows arrive in registers and the workgroup splits
+//     them into the LDS stage itself.  A wave's load takes 16 rows x 64 bytes (four lanes per row:
+//     full 64-byte requests), which its LDS writes then scatter without bank conflicts; with one
+//     load per 512 contiguous bytes of two rows, 16 lanes of every write met on the same banks
+//     (0.9 us of a 2.2 us stage).
 // Padding blocks (k is padded to 256) have scale 0 and x 0; a stage wholly past k is not run.
-constexpr int kQ8StageBlocks = 4;
-constexpr int kQ8StageK = kQ8StageBlocks * kQ8Block;
+//
+// Stores.  The accumulators go through LDS (rows of 36 floats per wave, the x buffers' space) so
+// that a lane stores 16 bytes: 4-byte stores cost the same address cycles each, four times as many
+// (1.9 -> 0.5 us at the end of a 64 x 128 tile).
+//
+// PAIR: a SwiGLU pair (Q8Group swiglu), a form of its own so the other calls carry none of it: the
+// first NS / 2 slabs are the gate's, the others the up's over the same columns.
+// GRP = false: one weight set (set 0), without the choice of a set.
+constexpr int kQ8OutLd = 36; // floats per row of a wave's 32-column output tile in LDS (16-byte rows, spread banks)
 
-// KS = 2: the workgroup's waves form two groups of NW, each over the same slabs and half of the
-// workgroup's stages (contiguous, each half a whole number of 2-stage turns), with x buffers of
-// their own; at the end the second group adds its sums into the first's through LDS (in that
-// order, so the result is the two halves' sums added once, as a 2-way k split would add them) and
-// the first stores.  For calls whose weight rows give too few workgroups for the chip and are not
-// split: each wave then walks half the stages, and two waves share each SIMD, with no partial
-// sums in memory and no second launch.
-// PAIR: a SwiGLU pair (Q8Group swiglu), a form of its own so the other calls carry none of it.
-template <int MT, int S, int NW, bool XS, int KS = 1, bool PAIR = false>
-__global__ __launch_bounds__(64 * NW * KS) __attribute__((amdgpu_waves_per_eu(2)))
-void linear_q8p_stream_kernel(Q8Args a, Q8Group grp, const _Float16 *xcvt) {
-    static_assert(KS == 1 || KS == 2, "one or two stage groups");
-    constexpr int NB = kQ8StageBlocks;
-    constexpr int NT = 64 * NW;                   // threads of one stage group
-    constexpr int SLABS = NW * S;                 // slabs of 32 weight rows per workgroup (NW waves)
-    constexpr int PIECES = NB * MT * 4;           // 1 KB pieces of an x stage
-    constexpr int XL = PIECES / NW;               // pieces each wave copies (XS = false)
-    static_assert(PIECES % NW == 0, "every wave copies whole pieces of the x stage");
-    constexpr int STAGE_HALVES = PIECES * 512;
-    constexpr int XQ = XS ? MT * 32 * kQ8StageK / 4 / NT : 1; // 16-byte x loads per thread (XS = true)
-    static_assert(!XS || XQ * 4 * NT == MT * 32 * kQ8StageK, "every thread loads whole quads of the x stage");
-    __shared__ __align__(16) _Float16 xs_all[KS][2][STAGE_HALVES];
+template <int MT, int NS, int MS, int KB, int SB, bool XS, bool PAIR, bool GRP>
+struct Q8pTile {
+    static constexpr int NW = NS * MS * KB;           // waves
+    static constexpr int NB = SB / KB;                // blocks of a stage per wave
+    static constexpr int WT = MT / MS;                // m-tiles per wave
+    static constexpr int K = SB * kQ8Block;           // k per stage
+    static constexpr int SPC = kQ8Chunk / K;          // stages per chunk
+    static constexpr int PIECES = SB * MT * 4;        // 1 KB pieces of an x stage
+    static constexpr int XL = PIECES / NW;            // pieces each wave copies (XS = false)
+    static constexpr int STAGE_HALVES = PIECES * 512; // one x stage in LDS
+    // XS: the x stage's quads go to the waves by groups of 16 rows (RG of them) x 16 k; CW waves
+    // share a row group's 2 SB column groups
+    static constexpr int RG = 2 * MT, CW = NW / RG;
+    static constexpr int XQ = XS ? 2 * SB / CW : 1;
+    static_assert(PIECES % NW == 0 && NW % RG == 0 && (2 * SB) % CW == 0 && MT % MS == 0, "x stage divides among the waves");
+    static constexpr int OT = WT * 32 * kQ8OutLd; // floats of one wave's output tile
+    static constexpr int OUT_BYTES = NW * OT * 4;
+    static constexpr int HS = NS / 2;
+    static constexpr int OS = PAIR ? HS : NS;   // output slabs
+    static constexpr int PW = OS * MT * 4 / NW; // pieces of 8 rows x 32 columns each wave stores
+    static constexpr int WPS = NW / OS;         // waves per output slab
+    static_assert(PW >= 1 && WPS * OS == NW && PW * WPS == MT * 4, "whole pieces per wave, one slab each");
+    static constexpr int NP = PAIR ? 2 : 1;
+    // the packed weights are streamed past the caches when nothing reads them again (32-row calls);
+    // a 64-row call's row blocks do, and its loads run at twice the rate per CU without the policy
+    // (a 1001 x 1536 x 8960 call 85 -> 71 us, the 64-row logits of 151936 rows 82 -> 79 us; the
+    // one-row logits 31 us with it, 33 without)
+    static constexpr int POLICY = MT == 1 ? kQ8CachePolicyNT : 0;
 
-    const int lane = threadIdx.x & 63;
-    const int wave_all = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); // uniform: the LDS DMA base is per wave
-    const int kg = KS == 1 ? 0 : wave_all / NW;                    // stage group
-    const int wave = KS == 1 ? wave_all : wave_all - kg * NW;      // wave within the group: its slabs
-    // this wave's weight set and its workgroup's index within the set.  A SwiGLU pair: the first
-    // NW / 2 waves take the gate's slabs and the others the up's slabs over the same columns.
-    constexpr bool pair = PAIR;
-    constexpr int HW = NW / 2;
-    const int set = pair ? (wave >= HW ? 1 : 0) : q8_group_of_block(grp, (int)blockIdx.x);
-    const int bx = (int)blockIdx.x - (pair ? 0 : q8_pick(grp.block_start, set));
-    const Q8Packed w = {q8_pick(grp.q, set), q8_pick(grp.scales, set), q8_pick(grp.n_slabs, set), grp.n_chunks};
-    a.n = q8_pick(grp.n, set);
-    a.bias = q8_pick(grp.bias, set);
-    a.out = q8_pick(grp.out, set);
-    a.part = q8_pick(grp.part, set);
-    // a call of more rows than one x stage holds runs gridDim.z blocks of 32 MT rows (XS only):
-    // block z takes rows r0 = 32 MT z .. of x and of the outputs; the partial sums keep the whole
-    // call's [split][m][n] layout
-    const int m_all = a.m;
-    const int r0 = (int)blockIdx.z * MT * 32;
-    a.m = min(MT * 32, m_all - r0);
-    a.x += (int64_t)r0 * a.k;
-
-    const int tid = KS == 1 ? (int)threadIdx.x : (int)threadIdx.x - kg * NT; // thread within the group
-    _Float16(&xs)[2][STAGE_HALVES] = xs_all[kg];
-    const int r32 = lane & 31, g = lane >> 5;
-    const int hw = pair ? wave - set * HW : wave;   // the wave's place among its set's waves
-    const int slab0 = bx * (pair ? HW * S : SLABS) + hw * S; // this wave's first slab
-    const int split = blockIdx.y;
-    const int n_stages = (a.k + NB * kQ8Block - 1) / (NB * kQ8Block);
-    const int w_begin = split * a.chunks_per_split * 2;
-    const int w_end = min(w_begin + a.chunks_per_split * 2, n_stages);
-    // this group's stages (whole 2-stage turns for the first group, so both groups run as many
-    // turns and meet the same barriers)
-    const int half = KS == 1 ? w_end - w_begin : ((w_end - w_begin + 3) / 4) * 2;
-    const int t_begin = min(w_begin + kg * half, w_end);
-    const int t_end = KS == 1 ? w_end : min(t_begin + half, w_end);
-    const int turns = (half + 1) / 2; // 2-stage loop turns, the same in every group
-
-    // XS: x [m][k] f32, rows past m read as 0 (range), columns past k get an out-of-range offset;
-    // otherwise the call's split x chunks
-    const __amdgpu_buffer_rsrc_t x_src =
-        XS ? rsrc(a.x, (uint32_t)a.m * (uint32_t)a.k * 4u) : rsrc(xcvt, (uint32_t)w.n_chunks * 2u * (uint32_t)PIECES * 1024u);
-    // slabs past the matrix (the last workgroup's) read as 0
-    const int live = __builtin_amdgcn_readfirstlane(max(0, min(S, w.n_slabs - slab0)));
-    const int64_t slab_q = (int64_t)w.n_chunks * kQ8ChunkBlocks * 1024;
-    const int64_t slab_s = (int64_t)w.n_chunks * 32 * kQ8ChunkBlocks * 4;
-    const __amdgpu_buffer_rsrc_t q_src = rsrc(w.q + (int64_t)slab0 * slab_q, (uint32_t)(live * slab_q));
-    const __amdgpu_buffer_rsrc_t s_src =
-        rsrc(reinterpret_cast<const char *>(w.scales) + (int64_t)slab0 * slab_s, (uint32_t)(live * slab_s));
-
-    // XS: x quad e of this thread in a stage is row x_r0 + XR e, k 4 (tid % 32) of the stage; 32
-    // consecutive threads read 512 contiguous bytes of a row.  The per-lane part of the offset is
-    // one VGPR; the row step and the stage's k go in the scalar offset.  The quad's place in the
-    // A-operand order: block, k-step and half of a lane's 8 elements follow the column, the m-tile
-    // and lane the row.
-    constexpr int XR = NT / 32; // rows between a thread's quads
-    const int x_r0 = tid >> 5, x_c = 4 * (tid & 31);
-    const uint32_t x_lane = ((uint32_t)x_r0 * (uint32_t)a.k + (uint32_t)x_c) * 4u;
-    const uint32_t x_rstep = (uint32_t)XR * (uint32_t)a.k * 4u;
-    const int x_b = x_c >> 5, x_kb = x_c & 31;
-    const int x_s = (x_kb >> 3) & 1, x_j = x_kb & 7;
-
-    // stage t: its x (into LDS buffer `buf`, or into xr), then this wave's weights and scales into
-    // (wq, sc).  Past the last stage (t >= t_end) the same loads go out with out-of-range offsets:
-    // they return zeros without touching memory, and every path through the loop then has the same
-    // loads in flight, so the compiler's in-order wait counts stay exact.
-    auto issue = [&](int t, int buf, f32x4 (&xr)[XQ], u32x4 (&wq)[S][NB], f32x4 (&sc)[S]) {
-        const bool live_t = t < t_end;
-        if constexpr (XS) {
-            const uint32_t xv = live_t && t * kQ8StageK + x_c < a.k ? x_lane : kOutOfRange;
-#pragma unroll
-            for (int e = 0; e < XQ; ++e)
-                xr[e] = __builtin_bit_cast(
-                    f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                               x_src, (int)xv, (int)((uint32_t)e * x_rstep + (uint32_t)(t * kQ8StageK) * 4u), 0));
-        } else {
-#pragma unroll
-            for (int u = 0; u < XL; ++u) {
-                const int piece = wave + NW * u;
-                const uint32_t off = live_t ? (uint32_t)((t * PIECES + piece) * 1024 + lane * 16) : kOutOfRange;
-                __builtin_amdgcn_raw_ptr_buffer_load_lds(
-                    x_src, (__attribute__((address_space(3))) void *)(&xs[buf][piece * 512]), 16, off, 0, 0, 0);
-            }
-        }
-#pragma unroll
-        for (int s = 0; s < S; ++s) {
-#pragma unroll
-            for (int b = 0; b < NB; ++b) {
-                const uint32_t off = live_t ? (uint32_t)(s * slab_q + ((int64_t)(t * NB + b) * 64 + lane) * 16)
-                                            : kOutOfRange;
-                wq[s][b] = __builtin_bit_cast(
-                    u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_src, (int)off, 0, kQ8CachePolicyNT));
-            }
-            // scales of blocks 4 (t % 2) .. +4 of chunk t / 2, this lane's row
-            const uint32_t off =
-                live_t ? (uint32_t)(s * slab_s + (((t >> 1) * 32 + r32) * kQ8ChunkBlocks + 4 * (t & 1)) * 4)
-                       : kOutOfRange;
-            sc[s] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(s_src, (int)off, 0, kQ8CachePolicyNT));
-        }
+    struct Scales {
+        float s[NB];
     };
-    // XS: the stage's x quads, split into f16 hi/lo halves, into LDS buffer `buf` (a quad is half of
-    // one lane's 8-element piece)
-    auto put_x = [&](int buf, const f32x4 (&xr)[XQ]) {
-        if constexpr (XS) {
+
+    int lane, wave, ws, ms, kg, set, bx, slab, r0, m, m_all, n, k, split, n_split, t_begin, t_end;
+    uint32_t epi;
+    __amdgpu_buffer_rsrc_t x_src, q_src, s_src;
+    int x_r, x_p, x_g0;
+    uint32_t x_lane, w_lane, s_lane;
+    int o_s, o_r, o_c, col;
+    f32x4 bv[NP];
+
+    __device__ __forceinline__ Q8pTile(const Q8Args &a, const Q8Group &grp, const _Float16 *xcvt) {
+        lane = threadIdx.x & 63;
+        wave = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6); // uniform: the LDS DMA base is per wave
+        ws = wave % NS;
+        ms = wave / NS % MS;
+        kg = wave / (NS * MS);
+        constexpr bool pick = PAIR || GRP;
+        set = PAIR ? (ws >= HS ? 1 : 0) : GRP ? q8_group_of_block(grp, (int)blockIdx.x) : 0;
+        bx = (int)blockIdx.x - (PAIR || !GRP ? 0 : q8_pick(grp.block_start, set));
+        const uint8_t *q = pick ? q8_pick(grp.q, set) : grp.q[0];
+        const float *scales = pick ? q8_pick(grp.scales, set) : grp.scales[0];
+        const int n_slabs = pick ? q8_pick(grp.n_slabs, set) : grp.n_slabs[0];
+        n = pick ? q8_pick(grp.n, set) : grp.n[0];
+        k = a.k;
+        epi = a.epi;
+        // a call of more rows than one x stage holds runs gridDim.z blocks of 32 MT rows: block z
+        // takes rows r0 = 32 MT z .. of x and of the outputs; the partial sums keep the whole
+        // call's [split][m][n] layout
+        m_all = a.m;
+        r0 = (int)blockIdx.z * MT * 32;
+        m = min(MT * 32, m_all - r0);
+        slab = bx * (PAIR ? HS : NS) + (PAIR ? ws - set * HS : ws); // this wave's slab
+        split = blockIdx.y;
+        n_split = a.n_split;
+        const int n_stages = (a.k + K - 1) / K;
+        t_begin = split * a.chunks_per_split * SPC;
+        t_end = min(t_begin + a.chunks_per_split * SPC, n_stages); // at least one stage
+        // XS: x [m][k] f32, rows past m read as 0 (range), columns past k get an out-of-range offset;
+        // otherwise this row block's split x chunks
+        const uint32_t xc_bytes = (uint32_t)grp.n_chunks * (uint32_t)(SPC * PIECES) * 1024u;
+        x_src = XS ? rsrc(a.x + (int64_t)r0 * a.k, (uint32_t)m * (uint32_t)a.k * 4u)
+                   : rsrc(reinterpret_cast<const char *>(xcvt) + (int64_t)blockIdx.z * xc_bytes, xc_bytes);
+        // a slab past the matrix (in the last workgroup) reads as 0
+        const bool live = slab < n_slabs;
+        const uint32_t slab_q = (uint32_t)grp.n_chunks * kQ8ChunkBlocks * 1024u;
+        const uint32_t slab_s = (uint32_t)grp.n_chunks * 32u * kQ8ChunkBlocks * 4u;
+        q_src = rsrc(q + (live ? (int64_t)slab * slab_q : 0), live ? slab_q : 0u);
+        s_src = rsrc(reinterpret_cast<const char *>(scales) + (live ? (int64_t)slab * slab_s : 0), live ? slab_s : 0u);
+        // XS: quad e of this thread in a stage is row x_r, k 16 (x_g0 + e) + 4 x_p of the stage.  The
+        // per-lane part of the offset is one VGPR, the stage's k goes in the scalar offset
+        x_r = 16 * (wave % RG) + (lane >> 2);
+        x_p = lane & 3;
+        x_g0 = wave / RG * XQ;
+        x_lane = ((uint32_t)x_r * (uint32_t)a.k + 4u * (uint32_t)x_p) * 4u;
+        w_lane = (uint32_t)lane * 16u;
+        s_lane = (uint32_t)(lane & 31) * (kQ8ChunkBlocks * 4u);
+        // the output pieces of this wave: slab o_s, rows o_r + 8 p, this lane's four columns and their bias
+        o_s = wave / WPS;
+        o_r = (wave % WPS) * PW * 8 + (lane >> 3);
+        o_c = 4 * (lane & 7);
+        col = (bx * OS + o_s) * 32 + o_c;
+#pragma unroll
+        for (int j = 0; j < NP; ++j) {
+            const float *bias = a.n_split > 1 ? nullptr : PAIR ? grp.bias[j] : GRP ? q8_pick(grp.bias, set) : grp.bias[0];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) bv[j][e] = bias && col + e < n ? bias[col + e] : 0.f;
+        }
+    }
+
+    // the loads of stage t: x quad e (XS) or this wave's pieces into an LDS buffer, this wave's block
+    // b of its slab, and the stage's scales of this lane's row
+    __device__ __forceinline__ f32x4 load_x(int t, int e) const {
+        const int at = t * K + 16 * (x_g0 + e); // whole column groups: k % 32 == 0
+        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                             x_src, (int)x_lane, (int)(t < t_end && at < k ? (uint32_t)at * 4u : kOutOfRange), 0));
+    }
+    __device__ __forceinline__ void dma_x(int t, _Float16 *buf) const {
+#pragma unroll
+        for (int u = 0; u < XL; ++u) {
+            const int piece = wave + NW * u;
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(x_src, (__attribute__((address_space(3))) void *)(buf + piece * 512), 16,
+                                                     w_lane, t < t_end ? (uint32_t)((t * PIECES + piece) * 1024) : kOutOfRange, 0, 0);
+        }
+    }
+    __device__ __forceinline__ u32x4 load_w(int t, int b) const {
+        const uint32_t at = (uint32_t)(t * SB + kg * NB + b) * 1024u;
+        return __builtin_bit_cast(
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_src, (int)w_lane, (int)(t < t_end ? at : kOutOfRange), POLICY));
+    }
+    __device__ __forceinline__ Scales load_s(int t) const {
+        const uint32_t at = (uint32_t)(t / SPC) * (32u * kQ8ChunkBlocks * 4u) + 4u * (uint32_t)(t % SPC * SB + kg * NB);
+        const int so = (int)(t < t_end ? at : kOutOfRange);
+        if constexpr (NB == 4)
+            return __builtin_bit_cast(Scales, __builtin_amdgcn_raw_buffer_load_b128(s_src, (int)s_lane, so, POLICY));
+        else if constexpr (NB == 2)
+            return __builtin_bit_cast(Scales, __builtin_amdgcn_raw_buffer_load_b64(s_src, (int)s_lane, so, POLICY));
+        else
+            return __builtin_bit_cast(Scales, __builtin_amdgcn_raw_buffer_load_b32(s_src, (int)s_lane, so, POLICY));
+    }
+    // XS: quad e split into an LDS buffer (a quad is half of one lane's 8-element piece)
+    __device__ __forceinline__ void put_x(_Float16 *buf, int e, const f32x4 &v) const {
+        half4 hi, lo;
+        zwg_split::split4(v, hi, lo);
+        const int cg = x_g0 + e, l = (x_r & 31) + 32 * (cg & 1), i = x_r >> 5, s = x_p >> 1, j = 4 * (x_p & 1);
+        *reinterpret_cast<half4 *>(buf + q8_xs_at<MT>(cg >> 1, i, 0, s, l) + j) = hi;
+        *reinterpret_cast<half4 *>(buf + q8_xs_at<MT>(cg >> 1, i, 1, s, l) + j) = lo;
+    }
+    // x operands of (this wave's block b, its m-tile i): hi and lo of k-step 0, hi and lo of k-step 1
+    __device__ __forceinline__ void read_a(half8 (&A)[4], const _Float16 *buf, int b, int i) const {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int hl = 0; hl < 2; ++hl)
+                A[2 * s + hl] = *reinterpret_cast<const half8 *>(buf + q8_xs_at<MT>(kg * NB + b, ms * WT + i, hl, s, lane));
+    }
+
+    // The stores, through the output tiles in `lds` (which every wave is done with): the bias, then
+    // the partial sums, or the epilogue and the output
+    __device__ __forceinline__ void store(const f32x16 (&acc)[WT], float *lds, const Q8Group &grp) const {
+        const int r32 = lane & 31, g = lane >> 5;
+        float *tile = lds + wave * OT;
+        // register r of lane l: row 32 i + 8 (r / 4) + 4 (l / 32) + r % 4, column (weight row) l % 32
+#pragma unroll
+        for (int i = 0; i < WT; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) tile[(32 * i + 8 * (r >> 2) + 4 * g + (r & 3)) * kQ8OutLd + r32] = acc[i][r];
+        __syncthreads();
+        if (col >= n) return;
+        f32x4 v[NP][PW];
+#pragma unroll
+        for (int j = 0; j < NP; ++j)
+#pragma unroll
+            for (int p = 0; p < PW; ++p) {
+                const int row = o_r + 8 * p;
+                const float *at = lds + (o_s + j * HS + row / (32 * WT) * NS) * OT + row % (32 * WT) * kQ8OutLd + o_c;
+                f32x4 q = *reinterpret_cast<const f32x4 *>(at);
+#pragma unroll
+                for (int g2 = 1; g2 < KB; ++g2) q += *reinterpret_cast<const f32x4 *>(at + g2 * NS * MS * OT);
+                v[j][p] = q + bv[j];
+            }
+        const bool vec = n % 4 == 0; // rows 16-byte aligned
+        auto put = [&](float *o, f32x4 q) {
+            if (vec) *reinterpret_cast<f32x4 *>(o) = q;
+            else
+                for (int e = 0; e < 4 && col + e < n; ++e) o[e] = q[e];
+        };
+        const int64_t o_at = (int64_t)(r0 + o_r) * n + col;
+        if (n_split > 1) {
+#pragma unroll
+            for (int j = 0; j < NP; ++j) {
+                float *part = (PAIR ? grp.part[j] : GRP ? q8_pick(grp.part, set) : grp.part[0]) + (int64_t)split * m_all * n + o_at;
+#pragma unroll
+                for (int p = 0; p < PW; ++p)
+                    if (o_r + 8 * p < m) put(part + (int64_t)8 * p * n, v[j][p]);
+            }
+            return;
+        }
+        float *o = (GRP && !PAIR ? q8_pick(grp.out, set) : grp.out[0]) + o_at;
+        if constexpr (PAIR) {
+#pragma unroll
+            for (int p = 0; p < PW; ++p)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[0][p][e] = zwg_ew::silu_mul(v[0][p][e], v[1][p][e]);
+        } else if (epi == zwg_ew::kEpiAdd) { // every residual load before the first store
+            f32x4 res[PW];
+#pragma unroll
+            for (int p = 0; p < PW; ++p) {
+                const float *op = o + (int64_t)8 * p * n;
+                if (o_r + 8 * p >= m) continue;
+                if (vec) res[p] = *reinterpret_cast<const f32x4 *>(op);
+                else
+                    for (int e = 0; e < 4; ++e) res[p][e] = col + e < n ? op[e] : 0.f;
+            }
+#pragma unroll
+            for (int p = 0; p < PW; ++p) v[0][p] = res[p] + v[0][p];
+        } else if (epi == zwg_ew::kEpiGelu) {
+#pragma unroll
+            for (int p = 0; p < PW; ++p)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[0][p][e] = zwg_ew::gelu(v[0][p][e]);
+        }
+#pragma unroll
+        for (int p = 0; p < PW; ++p)
+            if (o_r + 8 * p < m) put(o + (int64_t)8 * p * n, v[0][p]);
+    }
+};
+
+// Short calls (a chunk or so of k per workgroup, about one workgroup per CU): nothing but the order
+// of a wave's own instructions hides latency.  Stages of 128 k, three LDS buffers: at stage t the
+// buffers of t and t + 1 are complete and t + 2's is being filled, so a call of one or two stages has
+// one barrier before its products and none after.  A stage is walked in units of one (block,
+// m-tile): while a unit's four MFMAs run, the wave reads the next unit's x operands, widens the next
+// block's weights, scales the previous unit's sums and (XS) splits its share of stage t + 2's x.
+// Left to the compiler, each operand was read directly before its MFMA.  Measured back to back with
+// weights from HBM, against one workgroup shape with a barrier per stage and 4-byte stores:
+// 32 x 768 x 768 in 3 splits 5.8 -> 4.6 us, 64 x 1536 x 1536 in 6 splits 9.1 -> 6.0 us, 256 x 896 x
+// 896 in 4 splits 9.4 -> 6.1 us (64-column tiles; 128-column ones 7.0 and 7.5 us).
+template <int MT, int NS, int MS, bool XS, bool PAIR, bool GRP>
+__global__ __launch_bounds__(64 * NS * MS) __attribute__((amdgpu_waves_per_eu(2)))
+void linear_q8p_short_kernel(Q8Args a, Q8Group grp, const _Float16 *xcvt) {
+    using Tile = Q8pTile<MT, NS, MS, 1, 4, XS, PAIR, GRP>;
+    constexpr int NB = 4, WT = Tile::WT, XQ = Tile::XQ, XL = Tile::XL, U = NB * WT;
+    constexpr int XS_BYTES = 3 * Tile::STAGE_HALVES * 2;
+    __shared__ __align__(16) char lds_all[XS_BYTES > Tile::OUT_BYTES ? XS_BYTES : Tile::OUT_BYTES];
+    auto &xs = *reinterpret_cast<_Float16(*)[3][Tile::STAGE_HALVES]>(lds_all);
+    const Tile w(a, grp, xcvt);
+
+    f32x16 acc[WT];
+#pragma unroll
+    for (int i = 0; i < WT; ++i) acc[i] = (f32x16){0};
+    f32x4 xr[XQ];
+    u32x4 wq[3][NB];
+    typename Tile::Scales sc[3];
+
+    // stage t in buffer and register set `c`.  more: stages past t + 1 may follow (the last ones
+    // load and put nothing)
+    auto stage = [&](int t, auto c_c, auto more_c) {
+        constexpr int c = decltype(c_c)::value, c2 = (c + 2) % 3;
+        constexpr bool more = decltype(more_c)::value;
+        if constexpr (!XS && more) w.dma_x(t + 2, xs[c2]);
+        half8 A[2][4]; // a unit's x operands
+        half8 W[2][2]; // a block's widened weights
+        f32x16 T[2];   // a unit's sums
+        auto widen = [&](int b) { // and reload the block's registers for stage t + 3
+            W[b & 1][0] = int8x8_to_half8(wq[c][b][0], wq[c][b][1]);
+            W[b & 1][1] = int8x8_to_half8(wq[c][b][2], wq[c][b][3]);
+            if (more) wq[c][b] = w.load_w(t + 3, b);
+        };
+        auto scale = [&](int u) {
+            const float s = sc[c].s[u / WT];
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[u % WT][r] = __builtin_fmaf(T[u & 1][r], s, acc[u % WT][r]);
+        };
+        w.read_a(A[0], xs[c], 0, 0);
+        widen(0);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const half8(&au)[4] = A[u & 1];
+            const half8(&wu)[2] = W[(u / WT) & 1];
+            f32x16 tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(au[0], wu[0], (f32x16){0}, 0, 0, 0);
+            if (u + 1 < U) w.read_a(A[(u + 1) & 1], xs[c], (u + 1) / WT, (u + 1) % WT);
+            if (u % WT == WT - 1 && u / WT + 1 < NB) widen(u / WT + 1);
+            __builtin_amdgcn_sched_barrier(0);
+            tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(au[1], wu[0], tt, 0, 0, 0);
+            if (XS && more) { // a share of stage t + 2's x into LDS, its registers reloaded for t + 3
+#pragma unroll
+                for (int e = u * XQ / U; e < (u + 1) * XQ / U; ++e) {
+                    w.put_x(xs[c2], e, xr[e]);
+                    xr[e] = w.load_x(t + 3, e);
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(au[2], wu[1], tt, 0, 0, 0);
+            if (u > 0) scale(u - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            T[u & 1] = __builtin_amdgcn_mfma_f32_32x32x16_f16(au[3], wu[1], tt, 0, 0, 0);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        scale(U - 1);
+        if (more) sc[c] = w.load_s(t + 3);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (more) {
+            // XS = false: the copies of stage t + 1 (issued a stage ago) are whole, those of t + 2 and the
+            // loads after them may still be in flight
+            if constexpr (!XS) __builtin_amdgcn_s_waitcnt(q8_vmcnt(XL + 2 * (NB + 1)));
+            __syncthreads();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+
+    // first loads: x of stages 0 and 1, their weights and scales, then stage 2's
+    f32x4 x0[XQ], x1[XQ];
+    if constexpr (XS) {
+#pragma unroll
+        for (int e = 0; e < XQ; ++e) x0[e] = w.load_x(w.t_begin, e);
+#pragma unroll
+        for (int e = 0; e < XQ; ++e) x1[e] = w.load_x(w.t_begin + 1, e);
+    } else {
+        w.dma_x(w.t_begin, xs[0]);
+        w.dma_x(w.t_begin + 1, xs[1]);
+    }
+#pragma unroll
+    for (int c = 0; c < 2; ++c) {
+#pragma unroll
+        for (int b = 0; b < NB; ++b) wq[c][b] = w.load_w(w.t_begin + c, b);
+        sc[c] = w.load_s(w.t_begin + c);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (XS) {
+#pragma unroll
+        for (int e = 0; e < XQ; ++e) xr[e] = w.load_x(w.t_begin + 2, e);
+    }
+#pragma unroll
+    for (int b = 0; b < NB; ++b) wq[2][b] = w.load_w(w.t_begin + 2, b);
+    sc[2] = w.load_s(w.t_begin + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (XS) {
+#pragma unroll
+        for (int e = 0; e < XQ; ++e) w.put_x(xs[0], e, x0[e]);
+#pragma unroll
+        for (int e = 0; e < XQ; ++e) w.put_x(xs[1], e, x1[e]);
+    } else {
+        __builtin_amdgcn_s_waitcnt(q8_vmcnt(3 * (NB + 1)));
+    }
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    // turns of three stages, then the remaining one or two: the loop has no other way out, so the
+    // wait counts at its top are those of its own loads
+    const int n_t = w.t_end - w.t_begin;
+    int t = w.t_begin;
+    constexpr std::integral_constant<int, 0> c0{};
+    constexpr std::integral_constant<int, 1> c1{};
+    constexpr std::integral_constant<int, 2> c2{};
+    for (int p = n_t / 3; p > 0; --p, t += 3) {
+        stage(t, c0, std::true_type{});
+        stage(t + 1, c1, std::true_type{});
+        stage(t + 2, c2, std::true_type{});
+    }
+    if (n_t % 3 > 0) stage(t, c0, std::false_type{});
+    if (n_t % 3 > 1) stage(t + 1, c1, std::false_type{});
+    if constexpr (!XS) __builtin_amdgcn_s_waitcnt(q8_vmcnt(0)); // the last, out-of-range copies into LDS
+    __syncthreads();
+    w.store(acc, reinterpret_cast<float *>(lds_all), grp);
+}
+
+// Long calls (many stages per workgroup, or more workgroups than CUs): small stages of 64 k in two
+// LDS buffers, so that three or four 4-wave workgroups share a CU and hide each other's loads,
+// operand reads, first loads and stores.  Weights run two stages ahead in two register sets (block
+// b's registers are reloaded as soon as they are widened), x one stage.  Such a call is bound by the
+// bytes a CU can load (about 90-100 GB/s from L2 or the Infinity Cache, 32 KB of x and 16 KB of
+// weights per 64 x 128 x 128 products) with the MFMAs close behind; stages of 128 k, three or four
+// buffers, and eight-wave workgroups measured the same or slower.  Measured back to back, against
+// 128 k stages with a barrier, an LDS round trip per operand and 4-byte stores: the 64-row
+// logits of 151936 x 1536 91 -> 79 us, a 256-row SwiGLU pair of 4864 x 896 37 -> 20 us, the one-row
+// logits of 151936 x 896 58 -> 31 us, 1001 x 1536 x 8960 (the tiled kernel before) 120 -> 71 us.
+template <int MT, int NS, int KB, int SB, bool XS, bool PAIR, bool GRP>
+__global__ __launch_bounds__(64 * NS * KB) __attribute__((amdgpu_waves_per_eu(SB == 2 ? 3 : 2)))
+void linear_q8p_long_kernel(Q8Args a, Q8Group grp, const _Float16 *xcvt) {
+    using Tile = Q8pTile<MT, NS, 1, KB, SB, XS, PAIR, GRP>;
+    constexpr int WT = Tile::WT, XQ = Tile::XQ, NB = Tile::NB;
+    constexpr int XS_BYTES = 2 * Tile::STAGE_HALVES * 2;
+    __shared__ __align__(16) char lds_all[XS_BYTES > Tile::OUT_BYTES ? XS_BYTES : Tile::OUT_BYTES];
+    auto &xs = *reinterpret_cast<_Float16(*)[2][Tile::STAGE_HALVES]>(lds_all);
+    const Tile w(a, grp, xcvt);
+
+    f32x16 acc[WT];
+#pragma unroll
+    for (int i = 0; i < WT; ++i) acc[i] = (f32x16){0};
+    f32x4 xr[XQ]; // XS: the next stage's x
+    u32x4 wq[2][NB];
+    typename Tile::Scales sc[2];
+
+    // stage t in buffer and register set `c`; more: stages may follow
+    auto stage = [&](int t, auto c_c, auto more_c) {
+        constexpr int c = decltype(c_c)::value;
+        constexpr bool more = decltype(more_c)::value;
+        if constexpr (!XS && more) w.dma_x(t + 1, xs[c ^ 1]);
+        if constexpr (XS && more) {
 #pragma unroll
             for (int e = 0; e < XQ; ++e) {
-                const int row = x_r0 + XR * e;
-                const int i = row >> 5, l = (row & 31) + 32 * (x_kb >> 4);
-                half4 hi, lo;
-#pragma unroll
-                for (int c = 0; c < 4; ++c) {
-                    hi[c] = (_Float16)xr[e][c];
-                    lo[c] = (_Float16)(xr[e][c] - (float)hi[c]);
-                }
-                *reinterpret_cast<half4 *>(&xs[buf][q8_xs_at<MT>(x_b, i, 0, x_s, l) + x_j]) = hi;
-                *reinterpret_cast<half4 *>(&xs[buf][q8_xs_at<MT>(x_b, i, 1, x_s, l) + x_j]) = lo;
+                w.put_x(xs[c ^ 1], e, xr[e]);
+                xr[e] = w.load_x(t + 2, e);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
-    };
-
-    f32x16 acc[MT][S];
-#pragma unroll
-    for (int i = 0; i < MT; ++i)
-#pragma unroll
-        for (int s = 0; s < S; ++s) acc[i][s] = (f32x16){0};
-
-    auto compute = [&](int buf, const u32x4 (&wq)[S][NB], const f32x4 (&sc)[S]) {
 #pragma unroll
         for (int b = 0; b < NB; ++b) {
-            half8 ah[MT][2], al[MT][2];
+            const half8 w0 = int8x8_to_half8(wq[c][b][0], wq[c][b][1]);
+            const half8 w1 = int8x8_to_half8(wq[c][b][2], wq[c][b][3]);
+            if (more) wq[c][b] = w.load_w(t + 2, b);
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
+            for (int i = 0; i < WT; ++i) {
+                half8 A[4];
+                w.read_a(A, xs[c], b, i);
+                f32x16 tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[0], w0, (f32x16){0}, 0, 0, 0);
+                tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[1], w0, tt, 0, 0, 0);
+                tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[2], w1, tt, 0, 0, 0);
+                tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(A[3], w1, tt, 0, 0, 0);
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    ah[i][s] = *reinterpret_cast<const half8 *>(&xs[buf][q8_xs_at<MT>(b, i, 0, s, lane)]);
-                    al[i][s] = *reinterpret_cast<const half8 *>(&xs[buf][q8_xs_at<MT>(b, i, 1, s, lane)]);
-                }
-#pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const half8 w0 = int8x8_to_half8(wq[s][b][0], wq[s][b][1]);
-                const half8 w1 = int8x8_to_half8(wq[s][b][2], wq[s][b][3]);
-                const float scb = sc[s][b];
-#pragma unroll
-                for (int i = 0; i < MT; ++i) {
-                    f32x16 tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i][0], w0, (f32x16){0}, 0, 0, 0);
-                    tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i][0], w0, tt, 0, 0, 0);
-                    tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i][1], w1, tt, 0, 0, 0);
-                    tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(al[i][1], w1, tt, 0, 0, 0);
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i][s][r] = __builtin_fmaf(tt[r], scb, acc[i][s][r]);
-                }
+                for (int r = 0; r < 16; ++r) acc[i][r] = __builtin_fmaf(tt[r], sc[c].s[b], acc[i][r]);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
+        if (more) sc[c] = w.load_s(t + 2);
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (more) {
+            // XS = false: the copies of stage t + 1; the weights and scales issued after them may still
+            // be in flight
+            if constexpr (!XS) __builtin_amdgcn_s_waitcnt(q8_vmcnt(NB + 1));
+            __syncthreads();
+        }
+        __builtin_amdgcn_sched_barrier(0);
     };
 
-    // Two weight and scale register sets (A for even stages, B for odd) so every index is static;
-    // with XS one x register set, written into LDS at the top of its stage and then reloaded.
-    f32x4 xr[XQ];
-    u32x4 wqA[S][NB], wqB[S][NB];
-    f32x4 scA[S], scB[S];
-    constexpr int LOADS = S * (NB + 1); // weight and scale loads of one stage, issued after its x
-    issue(t_begin, 0, xr, wqA, scA);
-    for (int turn = 0, t = t_begin; KS == 1 ? t < t_end : turn < turns; ++turn, t += 2) {
-        // stage t (set A, buffer 0)
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(q8_vmcnt(LOADS));
-        put_x(0, xr);
-        __syncthreads();
-        __builtin_amdgcn_sched_barrier(0);
-        issue(t + 1, 1, xr, wqB, scB);
-        __builtin_amdgcn_sched_barrier(0);
-        if (KS == 1 || t < t_end) compute(0, wqA, scA); // the second group's may be empty
-        // stage t + 1 (set B, buffer 1); a no-op past the end (its loads returned zeros)
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(q8_vmcnt(LOADS));
-        put_x(1, xr);
-        __syncthreads();
-        __builtin_amdgcn_sched_barrier(0);
-        issue(t + 2, 0, xr, wqA, scA);
-        __builtin_amdgcn_sched_barrier(0);
-        if (t + 1 < t_end) compute(1, wqB, scB);
+    // first loads: stage 0's x, weights and scales, then stage 1's
+    f32x4 x0[XQ];
+    if constexpr (XS) {
+#pragma unroll
+        for (int e = 0; e < XQ; ++e) x0[e] = w.load_x(w.t_begin, e);
+    } else {
+        w.dma_x(w.t_begin, xs[0]);
     }
-    __builtin_amdgcn_s_waitcnt(q8_vmcnt(0)); // the last, out-of-range prefetch
-    if constexpr (KS == 2) {
-        // the second group's sums into the first's, through the (now free) x buffers: lane-major
-        // per (wave, m-tile, slab, register), conflict-free
-        float *red = reinterpret_cast<float *>(&xs_all[0][0][0]);
-        static_assert(NW * MT * S * 16 * 64 * 4 <= (int)sizeof(xs_all), "the sums fit in the x buffers");
-        __syncthreads(); // every wave is past its last compute
-        if (kg == 1) {
 #pragma unroll
-            for (int i = 0; i < MT; ++i)
+    for (int b = 0; b < NB; ++b) wq[0][b] = w.load_w(w.t_begin, b);
+    sc[0] = w.load_s(w.t_begin);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (XS) {
 #pragma unroll
-                for (int s = 0; s < S; ++s)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) red[(((wave * MT + i) * S + s) * 16 + r) * 64 + lane] = acc[i][s][r];
-        }
-        __syncthreads();
-        if (kg == 0) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int s = 0; s < S; ++s)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i][s][r] += red[(((wave * MT + i) * S + s) * 16 + r) * 64 + lane];
-        }
-        // an unsplit SwiGLU pair's second group stays for the barriers below
-        if (kg == 1 && !(PAIR && a.n_split == 1)) return;
+        for (int e = 0; e < XQ; ++e) xr[e] = w.load_x(w.t_begin + 1, e);
     }
-
-    // an unsplit SwiGLU pair: the up waves hand their values (with bias, as the call would store
-    // them) to the gate waves through the freed x buffers (past the two groups' exchange), which
-    // store silu(gate) * up
-    constexpr int RED2 = KS == 2 ? NW * MT * S * 16 * 64 : 0;
-    float *red = reinterpret_cast<float *>(&xs_all[0][0][0]) + RED2;
-    static_assert((RED2 + HW * MT * S * 16 * 64) * 4 <= (int)sizeof(xs_all), "the up values fit in the x buffers");
-    if (PAIR && a.n_split == 1) {
-        __syncthreads(); // every wave is past its last compute (and the first group's sums are whole)
-        if (kg == 0 && set == 1) {
 #pragma unroll
-            for (int s = 0; s < S; ++s) {
-                const int col = (slab0 + s) * 32 + r32;
-                const float bj = (a.bias && col < a.n) ? a.bias[col] : 0.f;
+    for (int b = 0; b < NB; ++b) wq[1][b] = w.load_w(w.t_begin + 1, b);
+    sc[1] = w.load_s(w.t_begin + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    if constexpr (XS) {
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) red[(((hw * MT + i) * S + s) * 16 + r) * 64 + lane] = acc[i][s][r] + bj;
-            }
-        }
-        __syncthreads();
-        if (kg == 1 || set == 1) return;
+        for (int e = 0; e < XQ; ++e) w.put_x(xs[0], e, x0[e]);
+    } else {
+        __builtin_amdgcn_s_waitcnt(q8_vmcnt(2 * (NB + 1)));
     }
-    float *dst = (a.n_split > 1 ? a.part + (int64_t)split * m_all * a.n : a.out) + (int64_t)r0 * a.n;
-#pragma unroll
-    for (int s = 0; s < S; ++s) {
-        const int col = (slab0 + s) * 32 + r32;
-        if (col >= a.n) continue;
-        const float bj = (a.n_split == 1 && a.bias) ? a.bias[col] : 0.f;
-        if (PAIR && a.n_split == 1) {
-#pragma unroll
-            for (int i = 0; i < MT; ++i)
-#pragma unroll
-                for (int r = 0; r < 16; ++r) {
-                    const int row = 32 * i + 8 * (r >> 2) + 4 * g + (r & 3);
-                    if (row < a.m)
-                        dst[(int64_t)row * a.n + col] =
-                            zwg_ew::silu_mul(acc[i][s][r] + bj, red[(((hw * MT + i) * S + s) * 16 + r) * 64 + lane]);
-                }
-            continue;
-        }
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int row = 32 * i + 8 * (r >> 2) + 4 * g + (r & 3);
-                if (row < a.m) {
-                    if (a.n_split > 1) dst[(int64_t)row * a.n + col] = acc[i][s][r];
-                    else zwg_ew::epilogue_store(&dst[(int64_t)row * a.n + col], acc[i][s][r] + bj, a.epi);
-                }
-            }
+    __syncthreads();
+    __builtin_amdgcn_sched_barrier(0);
+    // pairs of stages, then an odd one (the loop has no other way out, as above)
+    const int n_t = w.t_end - w.t_begin;
+    int t = w.t_begin;
+    for (int p = n_t / 2; p > 0; --p, t += 2) {
+        stage(t, std::integral_constant<int, 0>{}, std::true_type{});
+        stage(t + 1, std::integral_constant<int, 1>{}, std::true_type{});
     }
+    if (n_t & 1) stage(t, std::integral_constant<int, 0>{}, std::false_type{});
+    if constexpr (!XS) __builtin_amdgcn_s_waitcnt(q8_vmcnt(0)); // the last, out-of-range copies into LDS
+    __syncthreads();
+    w.store(acc, reinterpret_cast<float *>(lds_all), grp);
 }
 
 // out[i][o] (row stride ldo) = epilogue(sum over splits (in split order) of part[split][i][o],
