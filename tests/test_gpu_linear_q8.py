@@ -367,10 +367,11 @@ def test_two_stage_groups(torch, ctx, m, k, n):
 
 # One case per branch of the packed kernels' dispatch, at the edges of their tiles: one chunk of k per
 # workgroup (k split, 64-column tiles), several (128 or 256 columns), unsplit calls with fewer and more
-# 128-column units than CUs; one and two m-tiles and 64-row blocks with a ragged last one; n not a
+# 128-column units than CUs, calls of more than 256 rows on the packed kernels; one and two m-tiles and 64-row blocks with a ragged last one; n not a
 # multiple of 4 (4-byte stores), of 32 or of a tile; stage counts odd, even and past three.
 PACKED_CASES = [(1, 512, 70), (32, 288, 33), (31, 8960, 130), (33, 768, 257), (64, 8960, 1536), (129, 4864, 897),
-                (200, 1280, 4100), (48, 1376, 16386), (64, 544, 40004), (7, 480, 9001), (256, 96, 8200)]
+                (200, 1280, 4100), (48, 1376, 16386), (64, 544, 40004), (7, 480, 9001), (256, 96, 8200),
+                (300, 800, 4100), (1100, 3104, 1030)]
 
 
 @pytest.mark.parametrize("epilogue", ["none", "gelu", "add"])

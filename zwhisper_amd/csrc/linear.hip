@@ -70,7 +70,12 @@ TileChoice choose_tile(uint64_t m, uint64_t n) {
     } else {
         if (tiles(m, n, 128, 256) >= 512) return {128, 256};
     }
-    if (tiles(m, n, 64, 256) >= 256) return {64, 256};
+    if (tiles(m, n, 64, 256) >= 256) {
+        // a last column tile at most half full wastes more than the wider tile gains: 10000 x 384 x 384
+        // 19.0 -> 14.9 us, x 1536 x 384 53.7 -> 41.1; 24000 rows 29.4 -> 28.7 and 79.7 -> 80.2
+        if (WMODE == zwg_lin::kWF16 && (n - 1) % 256 < 128) return {128, 128};
+        return {64, 256};
+    }
     return {64, 64};
 }
 
@@ -79,6 +84,7 @@ hipError_t launch_tiled(const LinearArgs &a, TileChoice tc, int n_split, hipStre
     if constexpr (WMODE != zwg_lin::kWF16) {
         if (tc.bm == 128) return zwg_lin::launch_linear_tile<128, 128, WMODE>(a, n_split, stream);
     } else {
+        if (tc.bm == 128 && tc.bn == 128) return zwg_lin::launch_linear_tile<128, 128, WMODE, 4>(a, n_split, stream);
         if (tc.bm == 128) return zwg_lin::launch_linear_tile<128, 256, WMODE, 4>(a, n_split, stream);
     }
     if (tc.bn == 256) return zwg_lin::launch_linear_tile<64, 256, WMODE, 4>(a, n_split, stream);
@@ -348,8 +354,9 @@ hipError_t launch_q8p(const zwg_lin::Q8Args &a, const zwg_lin::Q8Group &g, const
         return launch_q8p_tile<false, 1, 4, 1, 4>(a, g, xcvt, XS, n_split, nz, st);
     } else {
         // one chunk per workgroup: 64 columns on four waves (64 x 1536 x 1536 in 6 splits 5.7, 128
-        // columns 6.6, the long kernel 6.9)
-        if (n_split > 1 && a.chunks_per_split == 1) return launch_q8p_tile<true, 2, 2, 2, 4>(a, g, xcvt, XS, n_split, nz, st);
+        // columns 6.6, the long kernel 6.9) while those, one per CU for their 96 KB of LDS, run at once
+        // (65 x 896 x 4864 in 4 splits, 608 of them: 19.6 with the split sum, the long kernel 14.5)
+        if (n_split > 1 && a.chunks_per_split == 1 && 2 * units * n_split <= 256) return launch_q8p_tile<true, 2, 2, 2, 4>(a, g, xcvt, XS, n_split, nz, st);
         // more units than CUs, split: 256 columns (256 x 4864 x 896 in 10 splits 14.5, 128 columns
         // 16.1); fewer: 128 columns (64 x 8960 x 1536 in 18 splits 12.0, 256 columns 13.9)
         if (n_split > 1 && units * n_split > 256) return launch_q8p_tile<false, 2, 8, 1, 2>(a, g, xcvt, XS, n_split, nz, st);
@@ -651,6 +658,18 @@ int run_q8w_token_step(zwg_ctx *ctx, const float *x, uint64_t m, uint32_t n_w, c
                   : run_q8p_group<1>(ctx, a, g, kvs, resln, po, xcvt_in);
 }
 
+// Calls of more than 256 rows that take the packed kernels (64-row blocks, unsplit) rather than the
+// tiled one: wide outputs, and long k with enough blocks to fill half the chip.  Measured against the
+// tiled kernel (its k split included): x 1536 x 8960 and x 896 x 4864 at 257 to 2048 rows 1.03 to 1.6
+// times as fast; 8960 x 1536 at 512 rows (96 blocks) 0.95, at 700 (132) 1.24; 4864 x 896 at 1001 rows
+// (112) 0.98, at 1500 (168) 1.23; 3072 x 768 at 1500 (144) 1.12; 512 x 2048 0.8 at any size.  The
+// split x needs room in the workspace.
+bool q8p_takes_rows(const zwg_ctx *ctx, uint64_t m, uint64_t k, uint64_t n) {
+    const uint64_t n_chunks = (k + zwg_lin::kQ8Chunk - 1) / zwg_lin::kQ8Chunk, nz = (m + 63) / 64;
+    if (nz > 65535 || nz * n_chunks * zwg_lin::q8_chunk_halves<2>() * 2 > ctx->workspace_bytes) return false;
+    return (n >= 4096 && k >= 768) || (k >= 3072 && nz * ((n + 127) / 128) >= 128);
+}
+
 int run_linear_q8w(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *w, const float *bias, float *out,
                    uint32_t epi) {
     if (!w) return fail(ctx, "null weights");
@@ -664,7 +683,7 @@ int run_linear_q8w(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *w, c
     if (!al16(x) || !al16(out)) return fail(ctx, "x and out must be 16-byte aligned");
     hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return fail_hip(ctx, "hipSetDevice", e);
-    if (m <= ZWG_Q8P_STREAM_ROWS) return run_q8w_token_step(ctx, x, m, 1, &w, &bias, &out, epi);
+    if (m <= ZWG_Q8P_STREAM_ROWS || q8p_takes_rows(ctx, m, w->k, w->n)) return run_q8w_token_step(ctx, x, m, 1, &w, &bias, &out, epi);
     LinearArgs a{};
     a.x = x;
     a.w = w->q;
