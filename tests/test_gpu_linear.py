@@ -187,3 +187,39 @@ def test_large_and_small_calls_agree_bitwise(torch, ctx, m, k, n):
         ctx.linear_epi_dev(xd[r0:r1].contiguous(), r1 - r0, k, wd, bd, n, small, _lib.EPI_NONE)
         torch.cuda.synchronize()
         assert torch.equal(small, big[r0:r1]), (r0, r1)
+
+
+@pytest.mark.parametrize("m,k,n,stride", [
+    (6000, 96, 384, 0),     # 64 x 64 tiles
+    (10001, 64, 384, 0),    # 128 x 128 tiles (a last column tile at most half full), a ragged row tile
+    (9000, 72, 512, 516),   # 64 x 256 tiles, a wider row stride
+    (9000, 72, 512, 514),   # rows not 16-byte aligned: 4-byte stores
+    (16400, 40, 2052, 0),   # 128 x 256 tiles, 135 MB of output: non-temporal stores, a partial column tile
+    (130, 1024, 200, 0),    # k split
+])
+@pytest.mark.parametrize("epilogue", ["none", "gelu", "add"])
+def test_store_paths(torch, ctx, m, k, n, stride, epilogue):
+    """Every epilogue of every tile's vector stores, against f64 (bar as above; GELU's slope is below 1.13),
+    and nothing written between the rows."""
+    from zwhisper_amd import _lib
+
+    x, w, b = inputs(m + k + n + stride, m, k, n)
+    ld = stride or n
+    g = torch.Generator(device="cuda").manual_seed(m + n)
+    old = torch.randn(m * ld, device="cuda", generator=g)
+    out = old.clone()
+    epi = {"none": _lib.EPI_NONE, "gelu": _lib.EPI_GELU, "add": _lib.EPI_ADD}[epilogue]
+    wd, bd = torch.from_numpy(w).cuda(), torch.from_numpy(b).cuda()
+    xd = torch.from_numpy(x).cuda()
+    ctx.linear_epi_dev(xd, m, k, wd, bd, n, out, epi, out_stride=stride)
+    ref = xd.double() @ wd.double().T + bd.double()
+    if epilogue == "gelu":
+        ref = 0.5 * ref * (1.0 + torch.tanh(0.7978845608028654 * (ref + 0.044715 * ref ** 3)))
+    elif epilogue == "add":
+        ref = ref + old.view(m, ld)[:, :n].double()
+    got = out.view(m, ld)
+    err = float((got[:, :n].double() - ref).abs().max())
+    bar = 1.13 * 2e-5 * np.sqrt(k)
+    print(f"linear {m}x{k}x{n} stride {ld} {epilogue}: max abs {err:.2e} (bar {bar:.1e})", flush=True)
+    assert bool(torch.isfinite(got).all()) and err <= bar
+    assert torch.equal(got[:, n:], old.view(m, ld)[:, n:])

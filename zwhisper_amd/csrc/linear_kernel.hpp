@@ -50,6 +50,8 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BK = 32;                 // K per LDS stage: one 64-byte LDS row
+constexpr int kNonTemporal = 2;        // the buffer operations' cache policy bit nt
+typedef uint32_t u32x4_st __attribute__((ext_vector_type(4)));
 constexpr uint32_t kOutOfRange = 0x80000000u; // a buffer offset past every range the host allows
 
 // Weight formats of the tiled kernel.
@@ -131,9 +133,11 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
     static_assert(XL >= 1 && TM >= 1 && TN >= 1, "tile too small for the workgroup");
     static_assert(W_LOADS % 64 == 0, "w loads must cover whole waves");
 
-    __shared__ __align__(16) _Float16 xh[2][BM * BK];
-    __shared__ __align__(16) _Float16 xl[2][BM * BK];
-    __shared__ __align__(16) _Float16 ws[2][BN * BK];
+    constexpr int kStage = 2 * BM * BK + BN * BK; // halves of one stage: x hi, x lo, w
+    __shared__ __align__(16) _Float16 lds[2 * kStage];
+    const auto xh = [&](int buf) { return lds + buf * kStage; };
+    const auto xl = [&](int buf) { return lds + buf * kStage + BM * BK; };
+    const auto ws = [&](int buf) { return lds + buf * kStage + 2 * BM * BK; };
 
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -209,14 +213,10 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
             const int f = tid + kThreads * i;
             const int row = f / (BK / 4), q = f % (BK / 4);
             half4 hi, lo;
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                hi[j] = (_Float16)xr[i][j];
-                lo[j] = (_Float16)(xr[i][j] - (float)hi[j]);
-            }
+            zwg_split::split4(xr[i], hi, lo);
             const int at = lds_at(row, q >> 1) + 4 * (q & 1);
-            *reinterpret_cast<half4 *>(&xh[buf][at]) = hi;
-            *reinterpret_cast<half4 *>(&xl[buf][at]) = lo;
+            *reinterpret_cast<half4 *>(&xh(buf)[at]) = hi;
+            *reinterpret_cast<half4 *>(&xl(buf)[at]) = lo;
         }
 #pragma unroll
         for (int i = 0; i < WL; ++i) {
@@ -228,11 +228,11 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
                 const int row = WMODE == kWQ8P ? ((f >> 6) << 5) + (f & 31) : f >> 1;
                 const int c = WMODE == kWQ8P ? 2 * ((f >> 5) & 1) : 2 * (f & 1);
                 const uint32_t *u = reinterpret_cast<const uint32_t *>(&wr[i]);
-                *reinterpret_cast<half8 *>(&ws[buf][lds_at(row, c)]) = int8x8_to_half8(u[0], u[1]);
-                *reinterpret_cast<half8 *>(&ws[buf][lds_at(row, c + 1)]) = int8x8_to_half8(u[2], u[3]);
+                *reinterpret_cast<half8 *>(&ws(buf)[lds_at(row, c)]) = int8x8_to_half8(u[0], u[1]);
+                *reinterpret_cast<half8 *>(&ws(buf)[lds_at(row, c + 1)]) = int8x8_to_half8(u[2], u[3]);
             } else {
                 const int row = f / (BK / 8), c = f % (BK / 8);
-                *reinterpret_cast<half8 *>(&ws[buf][lds_at(row, c)]) = __builtin_bit_cast(half8, wr[i]);
+                *reinterpret_cast<half8 *>(&ws(buf)[lds_at(row, c)]) = __builtin_bit_cast(half8, wr[i]);
             }
         }
     };
@@ -252,12 +252,12 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
 #pragma unroll
                 for (int i = 0; i < TM; ++i) {
                     const int at = lds_at(wm * WM + i * 32 + r32, 2 * kk + ch);
-                    ah[i] = *reinterpret_cast<const half8 *>(&xh[buf][at]);
-                    al[i] = *reinterpret_cast<const half8 *>(&xl[buf][at]);
+                    ah[i] = *reinterpret_cast<const half8 *>(&xh(buf)[at]);
+                    al[i] = *reinterpret_cast<const half8 *>(&xl(buf)[at]);
                 }
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
-                    b[j] = *reinterpret_cast<const half8 *>(&ws[buf][lds_at(wn * WN + j * 32 + r32, 2 * kk + ch)]);
+                    b[j] = *reinterpret_cast<const half8 *>(&ws(buf)[lds_at(wn * WN + j * 32 + r32, 2 * kk + ch)]);
 #pragma unroll
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -277,15 +277,15 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
 #pragma unroll
                 for (int kk = 0; kk < 2; ++kk) {
                     const int at = lds_at(wm * WM + i * 32 + r32, 2 * kk + ch);
-                    ah[i][kk] = *reinterpret_cast<const half8 *>(&xh[buf][at]);
-                    al[i][kk] = *reinterpret_cast<const half8 *>(&xl[buf][at]);
+                    ah[i][kk] = *reinterpret_cast<const half8 *>(&xh(buf)[at]);
+                    al[i][kk] = *reinterpret_cast<const half8 *>(&xl(buf)[at]);
                 }
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
                 half8 b[2];
 #pragma unroll
                 for (int kk = 0; kk < 2; ++kk)
-                    b[kk] = *reinterpret_cast<const half8 *>(&ws[buf][lds_at(wn * WN + j * 32 + r32, 2 * kk + ch)]);
+                    b[kk] = *reinterpret_cast<const half8 *>(&ws(buf)[lds_at(wn * WN + j * 32 + r32, 2 * kk + ch)]);
 #pragma unroll
                 for (int i = 0; i < TM; ++i) {
                     f32x16 t = __builtin_amdgcn_mfma_f32_32x32x16_f16(ah[i][0], b[0], (f32x16){0}, 0, 0, 0);
@@ -342,6 +342,75 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
             }
             return;
         }
+    }
+    // Rows of the output whose 16-byte groups are aligned go out 16 bytes per lane: each wave passes its
+    // 32 x 32 blocks through its own LDS tile (rows of 36 floats; a wave's LDS accesses stay in order,
+    // so no barrier) and stores 8 rows of 128 bytes at a time.  A 4-byte store costs the address unit
+    // as many cycles as a 16-byte one: 24000 x 512 x 2048 with GELU 136 -> 124 us, 1000 x 512 x 512
+    // with the residual add 10.1 -> 8.1, the other encoder shapes 1.01 to 1.3 times as fast.
+    constexpr int kLd = WN + 4, kCh = 32 / TN; // floats per tile row; rows of a chunk
+    constexpr int kLpr = WN / 4, kRpp = 64 / kLpr, kP = kCh / kRpp; // lanes per row, rows per piece, pieces
+    static_assert(TN == 1 || TN == 2, "a chunk's rows are whole register quads");
+    static_assert(2 * NWN * kCh * kLd * 4 <= 2 * kStage * 2, "the waves' tiles fit in the stages");
+    const int64_t ldd = KSPLIT ? a.n : a.ldo;
+    float *const dst = (KSPLIT ? a.part + (int64_t)split * a.m * a.n : a.out) + (int64_t)m0 * ldd + n0;
+    const int64_t dst_span = (int64_t)(min(BM, a.m - m0) - 1) * ldd + (a.n - n0); // elements from (m0, n0) on
+    if (ldd % 4 == 0 && a.n % 4 == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0 && dst_span < 0x1fffffffll) {
+        // A plain or GELU output of 128 MB or more (half the Infinity Cache) goes out non-temporal: its
+        // bursts of 16-byte stores would push out the x rows that the neighbouring column tiles re-read
+        // (24000 x 512 x 2048 with GELU, 197 MB, into alternating buffers: 146 us, 124 non-temporal).  A
+        // smaller one stays cached for the call that reads it next (base.en's layer over 4 windows,
+        // hidden rows of 49 MB: 205 us of the 4-byte kernel's 229, non-temporal 224 of 239).
+        const bool nt = !KSPLIT && (int64_t)a.m * a.n >= (32ll << 20);
+        const __amdgpu_buffer_rsrc_t o_dst = rsrc(dst, (uint32_t)(dst_span * 4));
+        __syncthreads(); // every wave is past its last operand read
+        float *const tile = reinterpret_cast<float *>(lds) + wave * kCh * kLd;
+        const int t_r = lane / kLpr, t_c = 4 * (lane % kLpr); // this lane's row and columns of a piece
+        const int row0 = wm * WM + t_r, col0 = wn * WN + t_c;
+        const bool add = !KSPLIT && a.epi == zwg_ew::kEpiAdd, gelu = !KSPLIT && a.epi == zwg_ew::kEpiGelu;
+        const bool col_in = n0 + col0 < a.n;
+        float bj[TN];
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int col = n0 + wn * WN + j * 32 + r32;
+            bj[j] = !KSPLIT && a.bias && col < a.n ? a.bias[col] : 0.f;
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            f32x4 res[TN][kP];
+            if (add) { // out + v: the row block's residual values before its first store
+#pragma unroll
+                for (int h = 0; h < TN; ++h)
+#pragma unroll
+                    for (int p = 0; p < kP; ++p) {
+                        const int row = row0 + i * 32 + h * kCh + kRpp * p;
+                        if (m0 + row < a.m && col_in) res[h][p] = *reinterpret_cast<const f32x4 *>(dst + row * ldd + col0);
+                    }
+            }
+#pragma unroll
+            for (int h = 0; h < TN; ++h) {
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16 / TN; ++r)
+                        tile[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * kLd + j * 32 + r32] = acc[i][j][h * (16 / TN) + r] + bj[j];
+#pragma unroll
+                for (int p = 0; p < kP; ++p) {
+                    f32x4 v = *reinterpret_cast<const f32x4 *>(tile + (t_r + kRpp * p) * kLd + t_c);
+                    if (add) v = res[h][p] + v;
+                    if (gelu)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) v[e] = zwg_ew::gelu(v[e]);
+                    const int row = row0 + i * 32 + h * kCh + kRpp * p;
+                    if (m0 + row >= a.m || !col_in) continue;
+                    if (KSPLIT || add || !nt) *reinterpret_cast<f32x4 *>(dst + row * ldd + col0) = v;
+                    else
+                        __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_st, v), o_dst, (int)((row * ldd + col0) * 4),
+                                                               0, kNonTemporal);
+                }
+            }
+        }
+        return;
     }
     if constexpr (!KSPLIT) {
         const int rows_o = min(BM, a.m - m0);
@@ -407,8 +476,11 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
     }
 }
 
+// The f16 64 x 256 tile is held to 80 VGPRs, three 8-wave workgroups per CU (its epilogue's residual
+// rows would take it to 82, two workgroups: 6000 x 384 x 1536 28.7 -> 33.2 us).
 template <int BM, int BN, int WMODE, int NWN = 2, bool KSPLIT = false>
-__global__ __launch_bounds__(128 * NWN) void linear_mfma_kernel(LinearArgs a) {
+__global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(WMODE == kWF16 && BM == 64 && BN == 256 ? 6 : 1)))
+void linear_mfma_kernel(LinearArgs a) {
     linear_mfma_body<BM, BN, WMODE, NWN, KSPLIT>(a);
 }
 
