@@ -636,7 +636,8 @@ void detach_q8w(void *obj) {
 int run_q8w_token_step(zwg_ctx *ctx, const float *x, uint64_t m, uint32_t n_w, const zwg_q8w *const *w,
                        const float *const *bias, float *const *out, uint32_t epi,
                        const zwg_lin::Q8KvStore *kvs = nullptr, const zwg_lin::Q8ResLn *resln = nullptr,
-                       Q8PartsOut *po = nullptr, const _Float16 *xcvt_in = nullptr, bool swiglu = false) {
+                       Q8PartsOut *po = nullptr, const _Float16 *xcvt_in = nullptr, bool swiglu = false,
+                       _Float16 *swiglu_xcvt = nullptr) {
     zwg_lin::Q8Args a{};
     a.x = x;
     a.m = (int32_t)m;
@@ -646,6 +647,7 @@ int run_q8w_token_step(zwg_ctx *ctx, const float *x, uint64_t m, uint32_t n_w, c
     zwg_lin::Q8Group g{};
     g.count = (int32_t)n_w;
     g.swiglu = swiglu ? 1 : 0;
+    g.xcvt_out = swiglu_xcvt;
     for (uint32_t j = 0; j < n_w; ++j) {
         g.q[j] = w[j]->q;
         g.scales[j] = w[j]->scales;
@@ -705,7 +707,7 @@ int run_linear_q8w(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *w, c
 
 int zwg_host::linear_q8w_qkv_kv(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *const *w,
                                 const float *const *bias, float *q_out, zwg_kv *kv, uint64_t layer, uint64_t seq0,
-                                const int32_t *pos_dev, int32_t *n_kv_out, int64_t pos0) {
+                                const int32_t *pos_dev, int32_t *n_kv_out, int64_t pos0, const _Float16 *xcvt_in) {
     if (!ctx) return fail(nullptr, "null context");
     if (!w || !kv) return fail(ctx, "null weight array or cache");
     if (kv->ctx != ctx) return fail(ctx, "the cache belongs to another context (or its context is closed)");
@@ -730,6 +732,7 @@ int zwg_host::linear_q8w_qkv_kv(zwg_ctx *ctx, const float *x, uint64_t m, const 
     if (rows && m > ZWG_Q8P_STREAM_ROWS) return fail(ctx, "one sequence's cache-writing q/k/v call takes at most 256 tokens");
     if (m == 0) return ZWG_OK;
     if (!x || !al16(x) || !q_out || !al16(q_out)) return fail(ctx, "x and q_out must be non-null and 16-byte aligned");
+    if (xcvt_in && (m <= 32 || !al16(xcvt_in))) return fail(ctx, "split rows are for calls of more than 32 rows (16-byte aligned)");
     const hipError_t e = hipSetDevice(ctx->device);
     if (e != hipSuccess) return fail_hip(ctx, "hipSetDevice", e);
     zwg_lin::Q8KvStore kvs{};
@@ -749,17 +752,17 @@ int zwg_host::linear_q8w_qkv_kv(zwg_ctx *ctx, const float *x, uint64_t m, const 
     kvs.d = (int32_t)d.d;
     kvs.pos0 = rows ? (int32_t)pos0 : 0;
     kvs.seq_step = rows ? 0 : 1;
-    return run_q8w_token_step(ctx, x, m, 3, w, bias, nullptr, zwg_ew::kEpiNone, &kvs);
+    return run_q8w_token_step(ctx, x, m, 3, w, bias, nullptr, zwg_ew::kEpiNone, &kvs, nullptr, nullptr, xcvt_in);
 }
 
 // x += xin . W^T + bias and ln_out = the norm of x (layer norm with ln_w, ln_b, or RMS norm with
 // ln_w; eps) for a decode step's or a prompt batch's rows (m <= 256, n <= 4096): one stream launch and
 // linear_split_sum_add_ln_kernel; a call too short to split k (k <= 256) runs the add epilogue and
-// the norm as two launches, with the same results.  xcvt_out (33..64 rows): ln_out also split for
-// the next call (q8w_xcvt_halves(n) halves), which takes it as xcvt_in.
+// the norm as two launches, with the same results.  xcvt_out (more than 32 rows): ln_out also split
+// for the next call (q8w_xcvt_halves(m, n) halves), which takes it as xcvt_in.
 int zwg_host::linear_q8w_add_ln(zwg_ctx *ctx, const float *xin, uint64_t m, const zwg_q8w *w, const float *bias,
                                 float *x, const float *ln_w, const float *ln_b, float eps, float *ln_out, int norm,
-                                _Float16 *xcvt_out) {
+                                _Float16 *xcvt_out, const _Float16 *xcvt_in) {
     if (!w || !w->ctx) return fail(ctx, w ? kQ8wClosed : "null weights");
     const std::string msg = check_linear(m, w->k, ZWG_W_Q8, w->n);
     if (!msg.empty()) return fail(ctx, msg);
@@ -771,26 +774,17 @@ int zwg_host::linear_q8w_add_ln(zwg_ctx *ctx, const float *xin, uint64_t m, cons
     if (!xin || !x || !ln_w || (!rms && !ln_b) || !ln_out || !al16(xin) || !al16(x) || !al16(ln_w) ||
         (ln_b && !al16(ln_b)) || !al16(ln_out) || (bias && !al16(bias)))
         return fail(ctx, "null or unaligned buffer (all 16-byte aligned)");
-    if (xcvt_out && (m <= 32 || !al16(xcvt_out)))
-        return fail(ctx, "split rows for the next call are for 33..64-row steps (16-byte aligned)");
+    if ((xcvt_out || xcvt_in) && (m <= 32 || !al16(xcvt_out) || !al16(xcvt_in)))
+        return fail(ctx, "split rows are for calls of more than 32 rows (16-byte aligned)");
     if (w->n_chunks < 2) {
-        if (xcvt_out) return fail(ctx, "the split rows for the next call need k above 256");
+        if (xcvt_out || xcvt_in) return fail(ctx, "the split rows for the next call need k above 256");
         const int rc = run_linear_q8w(ctx, xin, m, w, bias, x, zwg_ew::kEpiAdd);
         if (rc != ZWG_OK) return rc;
         return rms ? rms_norm(ctx, x, m, w->n, ln_w, eps, ln_out) : layer_norm(ctx, x, m, w->n, ln_w, ln_b, eps, ln_out);
     }
     zwg_lin::Q8ResLn r{x, ln_w, ln_b, ln_out, eps, rms ? zwg_ew::kNormRms : zwg_ew::kNormLayer, xcvt_out};
     float *outs[1] = {x};
-    return run_q8w_token_step(ctx, xin, m, 1, &w, &bias, outs, zwg_ew::kEpiAdd, nullptr, &r);
-}
-
-bool zwg_host::q8w_group_reads_xcvt(uint64_t m, uint32_t n_w, const zwg_q8w *const *w) {
-    if (m <= 32 || m > 64 || n_w == 0 || n_w > (uint32_t)zwg_lin::kQ8MaxGroup) return false;
-    constexpr int kRows = q8p_unit<2>();
-    int64_t gx = 0;
-    for (uint32_t j = 0; j < n_w; ++j) gx += ((int64_t)w[j]->n + kRows - 1) / kRows;
-    const int n_chunks = (int)((w[0]->k + zwg_lin::kQ8Chunk - 1) / zwg_lin::kQ8Chunk);
-    return !q8p_splits_x_itself<2>(gx, n_chunks);
+    return run_q8w_token_step(ctx, xin, m, 1, &w, &bias, outs, zwg_ew::kEpiAdd, nullptr, &r, nullptr, xcvt_in);
 }
 
 uint64_t zwg_host::q8w_stream_rows() { return ZWG_Q8P_STREAM_ROWS; }
@@ -800,7 +794,7 @@ uint64_t zwg_host::q8w_stream_rows() { return ZWG_Q8P_STREAM_ROWS; }
 // split; the same values as the two projections' group call followed by the SiLU-mul kernel.
 // xcvt_in as for linear_q8w_group_xcvt.
 int zwg_host::linear_q8w_swiglu(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *gate, const zwg_q8w *up,
-                                float *out, const _Float16 *xcvt_in) {
+                                float *out, const _Float16 *xcvt_in, _Float16 *xcvt_out) {
     const auto al16 = [](const void *p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; };
     if (!gate || !up) return fail(ctx, "null weights");
     if (!gate->ctx || !up->ctx) return fail(ctx, kQ8wClosed);
@@ -809,16 +803,17 @@ int zwg_host::linear_q8w_swiglu(zwg_ctx *ctx, const float *x, uint64_t m, const 
     if (!msg.empty()) return fail(ctx, msg);
     if (m == 0) return ZWG_OK;
     if (m > ZWG_Q8P_STREAM_ROWS || !x || !out || !al16(x) || !al16(out) ||
-        (xcvt_in && (!al16(xcvt_in) || m <= 32 || m > 64)))
-        return fail(ctx, "a SwiGLU call: m <= 256, x and out 16-byte aligned, split rows for 33..64 rows");
+        ((xcvt_in || xcvt_out) && (!al16(xcvt_in) || !al16(xcvt_out) || m <= 32)) || (xcvt_out && gate->n % 128))
+        return fail(ctx, "a SwiGLU call: m <= 256, x and out 16-byte aligned, split rows for more than 32 rows, split "
+                         "outputs of whole 128 columns");
     const zwg_q8w *w[2] = {gate, up};
     float *outs[2] = {out, nullptr};
     return run_q8w_token_step(ctx, x, m, 2, w, nullptr, outs, zwg_ew::kEpiNone, nullptr, nullptr, nullptr, xcvt_in,
-                              true);
+                              true, xcvt_out);
 }
 
-uint64_t zwg_host::q8w_xcvt_halves(uint64_t k) {
-    return (k + zwg_lin::kQ8Chunk - 1) / zwg_lin::kQ8Chunk * (uint64_t)zwg_lin::q8_chunk_halves<2>();
+uint64_t zwg_host::q8w_xcvt_halves(uint64_t m, uint64_t k) {
+    return (m + 63) / 64 * ((k + zwg_lin::kQ8Chunk - 1) / zwg_lin::kQ8Chunk) * (uint64_t)zwg_lin::q8_chunk_halves<2>();
 }
 
 // A grouped token-step call (as zwg_linear_q8w_group_dev, m <= 64) whose x was split by the

@@ -102,6 +102,17 @@ __device__ __forceinline__ void q8_xs_store(_Float16 *xcvt, int row, int gk, f32
     *reinterpret_cast<half4 *>(base + q8_xs_at<MT>(b, i, 1, s, l) + j) = lo;
 }
 
+// One element of such a row: v at x[row][gk]
+template <int MT>
+__device__ __forceinline__ void q8_xs_store1(_Float16 *xcvt, int row, int gk, float v) {
+    const int c = gk / kQ8Chunk, b = gk % kQ8Chunk >> 5, kb = gk & 31;
+    const int s = (kb >> 3) & 1, j = kb & 7, i = row >> 5, l = (row & 31) + 32 * (kb >> 4);
+    _Float16 *base = xcvt + (int64_t)c * q8_chunk_halves<MT>();
+    const _Float16 hi = (_Float16)v;
+    base[q8_xs_at<MT>(b, i, 0, s, l) + j] = hi;
+    base[q8_xs_at<MT>(b, i, 1, s, l) + j] = (_Float16)(v - (float)hi);
+}
+
 // x f32 [m][k] -> xcvt f16 [blocks of 32 MT rows][n_chunks][chunk layout above]; rows >= m and columns
 // >= k are 0.  One thread per 4 consecutive k of one row.
 template <int MT>
@@ -270,6 +281,10 @@ struct Q8Group {
     // workgroup takes the same columns of both sets and the call stores silu(gate) * up into
     // out[0] (linear_q8p_stream_kernel; split calls through linear_split_sum_swiglu_kernel)
     int32_t swiglu;
+    // a SwiGLU pair of more than 32 rows: nullptr, or silu(gate) * up goes here split into f16 hi/lo
+    // halves for the next 64-row-block call (linear_q8_xprep_kernel's layout; n % 128 == 0, so every
+    // column its stages read is written) instead of into out[0]
+    _Float16 *xcvt_out;
 };
 
 // entry j of a group field, by selects on the uniform j (no dynamic indexing of the kernel-
@@ -558,6 +573,15 @@ struct Q8pTile {
             for (int p = 0; p < PW; ++p)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) v[0][p][e] = zwg_ew::silu_mul(v[0][p][e], v[1][p][e]);
+            if (MT == 2 && grp.xcvt_out) { // (split from the rounded product: the asm keeps the two apart)
+                _Float16 *xc = grp.xcvt_out + (int64_t)blockIdx.z * ((n + kQ8Chunk - 1) / kQ8Chunk) * q8_chunk_halves<2>();
+#pragma unroll
+                for (int p = 0; p < PW; ++p) {
+                    asm volatile("" : "+v"(v[0][p]));
+                    if (o_r + 8 * p < m) q8_xs_store<2>(xc, o_r + 8 * p, col, v[0][p]);
+                }
+                return;
+            }
         } else if (epi == zwg_ew::kEpiAdd) { // every residual load before the first store
             f32x4 res[PW];
 #pragma unroll
@@ -920,7 +944,15 @@ __global__ __launch_bounds__(256) void linear_split_sum_swiglu_kernel(Q8Group gr
         if (bias) s += bias[e % n];
         gu[set] = s;
     }
-    grp.out[0][e] = zwg_ew::silu_mul(gu[0], gu[1]);
+    float v = zwg_ew::silu_mul(gu[0], gu[1]);
+    if (!grp.xcvt_out) {
+        grp.out[0][e] = v;
+        return;
+    }
+    asm volatile("" : "+v"(v)); // split from the rounded product
+    const int row = (int)(e / n);
+    q8_xs_store1<2>(grp.xcvt_out + (int64_t)(row >> 6) * ((n + kQ8Chunk - 1) / kQ8Chunk) * q8_chunk_halves<2>(), row & 63,
+                    (int)(e % n), v);
 }
 
 // The q/k/v group's split sum with the cache append fused into its stores (set 0 q, 1 k, 2 v of a
@@ -1036,8 +1068,8 @@ struct Q8ResLn {
     float *ln_out; // [m][n]
     float eps;
     int32_t norm; // zwg_ew::kNormLayer or kNormRms (host side: which instantiation)
-    // nullptr, or the normalised rows also split into f16 hi/lo halves for the next 64-row call
-    // (linear_q8_xprep_kernel's layout and values, rows m .. 63 zero); the one-thread-per-column
+    // nullptr, or the normalised rows also split into f16 hi/lo halves for the next call of 64-row blocks
+    // (linear_q8_xprep_kernel's layout and values, the last block's rows past m zero); the one-thread-per-column
     // kernel only
     _Float16 *xcvt;
 };
@@ -1160,8 +1192,10 @@ __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(co
         __syncthreads();
         const int n_cols = (n + kQ8Chunk - 1) / kQ8Chunk * (kQ8Chunk / 4); // float4 columns of whole chunks
         if (c < n_cols) {
-            q8_xs_store<2>(r.xcvt, row, 4 * c, rowbuf[c]);
-            for (int z = row + m; z < 64; z += m) q8_xs_store<2>(r.xcvt, z, 4 * c, (f32x4){0.f, 0.f, 0.f, 0.f});
+            const int64_t per_z = (int64_t)(n_cols / (kQ8Chunk / 4)) * q8_chunk_halves<2>();
+            q8_xs_store<2>(r.xcvt + (row >> 6) * per_z, row & 63, 4 * c, rowbuf[c]);
+            for (int z = row + m; z < (m + 63) / 64 * 64; z += m)
+                q8_xs_store<2>(r.xcvt + (z >> 6) * per_z, z & 63, 4 * c, (f32x4){0.f, 0.f, 0.f, 0.f});
         }
     }
 }

@@ -13,15 +13,15 @@
 //     T = attention(Q, caches[0 .. pos])             decode kernel over transposed keys (+ merge)
 //     X += o(T); H = rmsNorm(X, ffn_norm)            stream + linear_split_sum_add_ln_wide_kernel
 //                                                    (RMS), which also splits H into f16 hi/lo
-//                                                    halves when the gate/up call reads a split x
+//                                                    halves for the next call (more than 32 rows)
 //     G = silu(gate(H)) * up(H)                      one stream launch over both weight sets, each
 //                                                    workgroup on the same columns of both (a
 //                                                    SwiGLU pair; + one split sum when k is split);
-//                                                    no x split launch of its own
+//                                                    G written split for the down projection
 //     X += down(G); H = next layer's attn_norm(X), or the output norm after the last layer
 //                                                    stream + the sum, residual add and norm
-//   logits = H . output^T                           one stream launch (33..64 sequences: x split by
-//                                                    the last down projection's sum kernel)
+//   logits = H . output^T                           one launch (33..64 sequences: x split by the
+//                                                    last down projection's sum kernel)
 //
 // The fused launches form the same values in the same order as the separate calls (the split
 // sums in split order, the residual add, zwg_ew::rms_norm_regs for every norm, the x split's f16
@@ -95,12 +95,21 @@ std::string check_llm(const zwg_ctx *ctx, const zwg_llm &lm, uint64_t n_seq_need
     return msg;
 }
 
+// Where a batch of m rows keeps its gated rows split for the down projection: in the m n_ff floats of
+// G and the m n_ff after them, which a split batch uses for nothing else; nullptr for batches of at
+// most 32 rows (split in the kernel), rows of broken 128-column stages (the split leaves their padding
+// unwritten), a down projection of one chunk, or where the blocks of 64 rows do not fit.
+_Float16 *gated_xcvt(float *G, uint64_t m, uint64_t nff) {
+    const bool fits = m > 32 && nff > 256 && nff % 128 == 0 && q8w_xcvt_halves(m, nff) / 2 <= 2 * m * nff;
+    return fits ? reinterpret_cast<_Float16 *>(G) : nullptr;
+}
+
 } // namespace
 
 extern "C" {
 
 uint64_t zwg_llm_scratch(uint64_t m, uint64_t n_embd, uint64_t n_ff) {
-    return 4 * m * n_embd + 2 * m * n_ff + (m + 3) / 4 * 4 + q8w_xcvt_halves(n_embd) / 2;
+    return 4 * m * n_embd + 2 * m * n_ff + (m + 3) / 4 * 4 + q8w_xcvt_halves(64, n_embd) / 2;
 }
 
 int zwg_llm_step_dev(zwg_ctx *ctx, const zwg_llm *lm, const int32_t *tokens, const int32_t *pos, uint64_t m,
@@ -121,8 +130,7 @@ int zwg_llm_step_dev(zwg_ctx *ctx, const zwg_llm *lm, const int32_t *tokens, con
     const int rms = zwg_ew::kNormRms;
     float *X = scratch, *Hn = X + m * ne, *Q = Hn + m * ne, *T = Q + m * ne, *G = T + m * ne, *U = G + m * nff;
     int32_t *n_kv = reinterpret_cast<int32_t *>(U + m * nff);
-    // the ffn-normed rows split for the gate/up call, when that call reads a split pass (written by
-    // the o projection's sum kernel, so the call needs no split launch of its own)
+    // the normed rows split for the call that reads them next
     _Float16 *xc = reinterpret_cast<_Float16 *>(reinterpret_cast<float *>(n_kv) + (m + 3) / 4 * 4);
     zwg_kv *kv = lm->kv;
     // src/llm.zig:175: embd.row, then the first block's attn_norm (:178)
@@ -150,34 +158,38 @@ int zwg_llm_step_dev(zwg_ctx *ctx, const zwg_llm *lm, const int32_t *tokens, con
     bt.out_bstride = ne;
     bt.n_kv_dev = n_kv;
 
-    const zwg_q8w *gu0[2] = {lm->layers[0].w_gate, lm->layers[0].w_up};
-    _Float16 *gu_xc = q8w_group_reads_xcvt(m, 2, gu0) ? xc : nullptr;
-    // likewise the output-normed rows for the logits, from the last down projection's sum kernel
-    _Float16 *out_xc = q8w_group_reads_xcvt(m, 1, &lm->output) ? xc : nullptr;
+    // Steps of more than 32 sequences hand each projection its rows already split for the matrix units:
+    // the norms' rows by the sum kernel that forms them, the gated rows (in G and U's place) by the
+    // gate/up call's own store when the down projection's stages are whole
+    const bool split = m > 32;
+    _Float16 *const n_xc = split && nff > 256 ? xc : nullptr; // written by the down projection's sum kernel
+    _Float16 *const g_xc = gated_xcvt(G, m, nff);
     for (uint64_t l = 0; l < lm->n_layer; ++l) {
         const zwg_llm_layer &L = lm->layers[l];
         // src/llm.zig:179-190: q/k/v, rotary positions, the cache writes
         const zwg_q8w *qkv[3] = {L.wq, L.wk, L.wv};
         const float *qkv_b[3] = {L.bq, L.bk, L.bv};
-        if ((rc = linear_q8w_qkv_kv(ctx, Hn, m, qkv, qkv_b, Q, kv, l, seq0, pos, n_kv)) != ZWG_OK) return rc;
+        if ((rc = linear_q8w_qkv_kv(ctx, Hn, m, qkv, qkv_b, Q, kv, l, seq0, pos, n_kv, -1, l ? n_xc : nullptr)) !=
+            ZWG_OK) return rc;
         const uint64_t at = (l * kv->desc.n_seq + seq0) * kv->per_seq;
         if ((rc = zwg_attention_batch_dev(ctx, Q, kv->k + at, kv->v + at, &sh, &bt, T)) != ZWG_OK) return rc;
         // :203-204 and the ffn norm (:206)
-        if ((rc = linear_q8w_add_ln(ctx, T, m, L.wo, nullptr, X, L.ffn_norm, nullptr, lm->eps, Hn, rms, gu_xc)) !=
+        if ((rc = linear_q8w_add_ln(ctx, T, m, L.wo, nullptr, X, L.ffn_norm, nullptr, lm->eps, Hn, rms,
+                                    split ? xc : nullptr)) !=
             ZWG_OK)
             return rc;
         // :207-211: gate and up, SiLU-gated, down, then the next block's attn_norm or the output
         // norm (:215)
-        if ((rc = linear_q8w_swiglu(ctx, Hn, m, L.w_gate, L.w_up, G, gu_xc)) != ZWG_OK) return rc;
+        if ((rc = linear_q8w_swiglu(ctx, Hn, m, L.w_gate, L.w_up, G, split ? xc : nullptr, g_xc)) != ZWG_OK) return rc;
         const bool last = l + 1 == lm->n_layer;
         const float *nw = last ? lm->output_norm : lm->layers[l + 1].attn_norm;
-        if ((rc = linear_q8w_add_ln(ctx, G, m, L.w_down, nullptr, X, nw, nullptr, lm->eps, Hn, rms,
-                                    last ? out_xc : nullptr)) != ZWG_OK)
+        if ((rc = linear_q8w_add_ln(ctx, G, m, L.w_down, nullptr, X, nw, nullptr, lm->eps, Hn, rms, n_xc,
+                                    g_xc)) != ZWG_OK)
             return rc;
     }
     // the logits of every sequence's token (src/llm.zig:216)
     float *outs[1] = {logits};
-    return linear_q8w_group_xcvt(ctx, Hn, m, 1, &lm->output, nullptr, outs, out_xc);
+    return linear_q8w_group_xcvt(ctx, Hn, m, 1, &lm->output, nullptr, outs, n_xc);
 }
 
 uint64_t zwg_llm_forward_scratch(uint64_t n, uint64_t n_embd, uint64_t n_ff) {
@@ -229,6 +241,11 @@ int zwg_llm_forward_dev(zwg_ctx *ctx, const zwg_llm *lm, const int32_t *tokens, 
     // decode step: the q/k/v projections writing the cache, and the residual projections' split
     // sums adding into x and normalising it for the next block, with the same results
     const bool fused = n <= q8w_stream_rows();
+    // and hand each projection its rows already split, as the decode step does (the norms' in the
+    // place of the separate calls' key and value rows), where the blocks of 64 rows fit
+    _Float16 *const xc = fused && n > 32 && q8w_xcvt_halves(n, ne) / 2 <= 2 * n * ne ? reinterpret_cast<_Float16 *>(Kb) : nullptr;
+    _Float16 *const n_xc = nff > 256 ? xc : nullptr;
+    _Float16 *const g_xc = fused ? gated_xcvt(G, n, nff) : nullptr;
     for (uint64_t l = 0; l < lm->n_layer; ++l) {
         const zwg_llm_layer &L = lm->layers[l];
         if (l > 0 && !fused && (rc = rms_norm(ctx, X, n, ne, L.attn_norm, lm->eps, Hn)) != ZWG_OK) return rc;
@@ -237,7 +254,8 @@ int zwg_llm_forward_dev(zwg_ctx *ctx, const zwg_llm *lm, const int32_t *tokens, 
         const float *qkv_b[3] = {L.bq, L.bk, L.bv};
         float *qkv_out[3] = {Q, Kb, Vb};
         if (fused) {
-            if ((rc = linear_q8w_qkv_kv(ctx, Hn, n, qkv, qkv_b, Q, kv, l, seq, nullptr, nullptr, (int64_t)pos0)) !=
+            if ((rc = linear_q8w_qkv_kv(ctx, Hn, n, qkv, qkv_b, Q, kv, l, seq, nullptr, nullptr, (int64_t)pos0,
+                                        l ? n_xc : nullptr)) !=
                 ZWG_OK)
                 return rc;
         } else {
@@ -249,14 +267,14 @@ int zwg_llm_forward_dev(zwg_ctx *ctx, const zwg_llm *lm, const int32_t *tokens, 
         if ((rc = zwg_attention_dev(ctx, Q, kv->k + at, kv->v + at, &sh, T)) != ZWG_OK) return rc;
         // :203-211
         if (fused) {
-            if ((rc = linear_q8w_add_ln(ctx, T, n, L.wo, nullptr, X, L.ffn_norm, nullptr, lm->eps, Hn, rms)) != ZWG_OK)
+            if ((rc = linear_q8w_add_ln(ctx, T, n, L.wo, nullptr, X, L.ffn_norm, nullptr, lm->eps, Hn, rms, xc)) != ZWG_OK)
                 return rc;
         } else {
             if ((rc = zwg_linear_q8w_epi_dev(ctx, T, n, L.wo, nullptr, X, ZWG_EPI_ADD)) != ZWG_OK) return rc;
             if ((rc = rms_norm(ctx, X, n, ne, L.ffn_norm, lm->eps, Hn)) != ZWG_OK) return rc;
         }
         if (fused) {
-            if ((rc = linear_q8w_swiglu(ctx, Hn, n, L.w_gate, L.w_up, G)) != ZWG_OK) return rc;
+            if ((rc = linear_q8w_swiglu(ctx, Hn, n, L.w_gate, L.w_up, G, xc, g_xc)) != ZWG_OK) return rc;
         } else {
             const zwg_q8w *gu[2] = {L.w_gate, L.w_up};
             float *gu_out[2] = {G, U};
@@ -266,7 +284,7 @@ int zwg_llm_forward_dev(zwg_ctx *ctx, const zwg_llm *lm, const int32_t *tokens, 
         if (fused) {
             // the next block's attn_norm, or the output norm (of every row; the logits take the last)
             const float *nw = l + 1 == lm->n_layer ? lm->output_norm : lm->layers[l + 1].attn_norm;
-            if ((rc = linear_q8w_add_ln(ctx, G, n, L.w_down, nullptr, X, nw, nullptr, lm->eps, Hn, rms)) != ZWG_OK)
+            if ((rc = linear_q8w_add_ln(ctx, G, n, L.w_down, nullptr, X, nw, nullptr, lm->eps, Hn, rms, n_xc, g_xc)) != ZWG_OK)
                 return rc;
         } else if ((rc = zwg_linear_q8w_epi_dev(ctx, G, n, L.w_down, nullptr, X, ZWG_EPI_ADD)) != ZWG_OK) {
             return rc;

@@ -91,27 +91,27 @@ int linear_q8w_parts(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *w,
 // zwg_linear_q8w_qkv_kv_dev with, when n_kv_out is set, each sequence's key count after the
 // append (pos + 1, 0 for a position off the cache) written to n_kv_out[m] by the same launch.
 // pos_dev nullptr: the m rows are one sequence's (seq0) tokens at pos0 .. pos0 + m - 1 (a prompt
-// batch, m <= q8w_stream_rows()).
+// batch, m <= q8w_stream_rows()).  xcvt_in (more than 32 rows): x as linear_q8w_add_ln split it.
 int linear_q8w_qkv_kv(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *const *w, const float *const *bias,
                       float *q_out, zwg_kv *kv, uint64_t layer, uint64_t seq0, const int32_t *pos_dev,
-                      int32_t *n_kv_out, int64_t pos0 = -1);
+                      int32_t *n_kv_out, int64_t pos0 = -1, const _Float16 *xcvt_in = nullptr);
 // rows up to which the int8 calls stream the resident weights (and the fused calls take)
 uint64_t q8w_stream_rows();
 // out = silu(x . gate^T) * (x . up^T), m <= q8w_stream_rows() (one stream launch over both sets);
-// xcvt_in as for linear_q8w_group_xcvt
+// xcvt_in (more than 32 rows): x as linear_q8w_add_ln split it; xcvt_out (likewise, n % 128 == 0): the
+// output goes there split for the next call (q8w_xcvt_halves(m, n) halves; rows past m unwritten) and
+// not to out
 int linear_q8w_swiglu(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *gate, const zwg_q8w *up, float *out,
-                      const _Float16 *xcvt_in = nullptr);
+                      const _Float16 *xcvt_in = nullptr, _Float16 *xcvt_out = nullptr);
 // A decode step's residual projection and the next norm: x += xin . W^T + bias, then ln_out =
 // the norm of x (norm 0: layer norm, 1: RMS norm; m <= q8w_stream_rows(), n <= 4096; linear.hip).  xcvt_out
-// (33..64 rows): ln_out also split into f16 hi/lo halves for the next call (q8w_xcvt_halves(n)
-// halves), passed to it as xcvt_in.
+// (more than 32 rows): ln_out also split into f16 hi/lo halves for the next call
+// (q8w_xcvt_halves(m, n) halves), passed to it as xcvt_in.  xcvt_in: xin's split, xin is not read.
 int linear_q8w_add_ln(zwg_ctx *ctx, const float *xin, uint64_t m, const zwg_q8w *w, const float *bias, float *x,
                       const float *ln_w, const float *ln_b, float eps, float *ln_out, int norm = 0,
-                      _Float16 *xcvt_out = nullptr);
-uint64_t q8w_xcvt_halves(uint64_t k);
-// whether a token-step group call of these weights over m rows streams its x from a split pass
-// (and so takes linear_q8w_group_xcvt's xcvt_in)
-bool q8w_group_reads_xcvt(uint64_t m, uint32_t n_w, const zwg_q8w *const *w);
+                      _Float16 *xcvt_out = nullptr, const _Float16 *xcvt_in = nullptr);
+// halves of m rows of k split for the packed int8 kernels (whole blocks of 64 rows, chunks of 256 k)
+uint64_t q8w_xcvt_halves(uint64_t m, uint64_t k);
 // zwg_linear_q8w_group_dev over rows whose split was written by linear_q8w_add_ln (xcvt_in)
 int linear_q8w_group_xcvt(zwg_ctx *ctx, const float *x, uint64_t m, uint32_t n_w, const zwg_q8w *const *w,
                           const float *const *bias, float *const *out, const _Float16 *xcvt_in);
