@@ -57,9 +57,10 @@ __device__ __forceinline__ float wave_sum(float v) {
 // differs from the reference's 16-lane vector order (a few f32 ulps).  Every kernel that normalises
 // a row goes through this function, so a fused norm equals the separate one bit for bit.
 // copy: nullptr, or a second destination of the output float4s (same index as in orow).
-template <int R>
-__device__ __forceinline__ void layer_norm_regs(const ew_f32x4 (&v)[R], int lane, int n4, const float *w,
-                                                const float *b, float eps, float *orow, ew_f32x4 *copy = nullptr) {
+// The norm weights (w, b: callables of i) may be loaded before the row is whole.
+template <int R, typename W, typename B>
+__device__ __forceinline__ void layer_norm_with(const ew_f32x4 (&v)[R], int lane, int n4, W w, B b, float eps, float *orow,
+                                                ew_f32x4 *copy) {
     const float fn = (float)(4 * n4);
     float s = 0.f;
 #pragma unroll
@@ -82,8 +83,7 @@ __device__ __forceinline__ void layer_norm_regs(const ew_f32x4 (&v)[R], int lane
     for (int i = 0; i < R; ++i) {
         const int c = lane + 64 * i;
         if (c < n4) {
-            const ew_f32x4 wv = reinterpret_cast<const ew_f32x4 *>(w)[c];
-            const ew_f32x4 bv = reinterpret_cast<const ew_f32x4 *>(b)[c];
+            const ew_f32x4 wv = w(i), bv = b(i);
             ew_f32x4 o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) o[e] = __builtin_fmaf((v[i][e] - mean) * inv, wv[e], bv[e]);
@@ -97,9 +97,9 @@ __device__ __forceinline__ void layer_norm_regs(const ew_f32x4 (&v)[R], int lane
 // x^2 (each lane's fmas, then a butterfly sum across the wave), inv = 1 / sqrt(ss / n + eps), out
 // = x * inv * w, multiplied left to right.  Every kernel that RMS-normalises a row goes through
 // this function.
-template <int R>
-__device__ __forceinline__ void rms_norm_regs(const ew_f32x4 (&v)[R], int lane, int n4, const float *w, float eps,
-                                              float *orow, ew_f32x4 *copy = nullptr) {
+template <int R, typename W>
+__device__ __forceinline__ void rms_norm_with(const ew_f32x4 (&v)[R], int lane, int n4, W w, float eps, float *orow,
+                                              ew_f32x4 *copy) {
     const float fn = (float)(4 * n4);
     float q = 0.f;
 #pragma unroll
@@ -115,7 +115,7 @@ __device__ __forceinline__ void rms_norm_regs(const ew_f32x4 (&v)[R], int lane, 
     for (int i = 0; i < R; ++i) {
         const int c = lane + 64 * i;
         if (c < n4) {
-            const ew_f32x4 wv = reinterpret_cast<const ew_f32x4 *>(w)[c];
+            const ew_f32x4 wv = w(i);
             ew_f32x4 o;
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
@@ -131,12 +131,42 @@ __device__ __forceinline__ void rms_norm_regs(const ew_f32x4 (&v)[R], int lane, 
 
 // The row norms of the fused kernels: layer norm (w, b) or RMS norm (w; b unused)
 constexpr int kNormLayer = 0, kNormRms = 1;
+template <int R>
+__device__ __forceinline__ void layer_norm_regs(const ew_f32x4 (&v)[R], int lane, int n4, const float *w, const float *b,
+                                                float eps, float *orow, ew_f32x4 *copy = nullptr) {
+    layer_norm_with<R>(v, lane, n4, [&](int i) { return reinterpret_cast<const ew_f32x4 *>(w)[lane + 64 * i]; },
+                       [&](int i) { return reinterpret_cast<const ew_f32x4 *>(b)[lane + 64 * i]; }, eps, orow, copy);
+}
+template <int R>
+__device__ __forceinline__ void rms_norm_regs(const ew_f32x4 (&v)[R], int lane, int n4, const float *w, float eps,
+                                              float *orow, ew_f32x4 *copy = nullptr) {
+    rms_norm_with<R>(v, lane, n4, [&](int i) { return reinterpret_cast<const ew_f32x4 *>(w)[lane + 64 * i]; }, eps, orow, copy);
+}
 template <int KIND, int R>
 __device__ __forceinline__ void norm_regs(const ew_f32x4 (&v)[R], int lane, int n4, const float *w, const float *b,
                                           float eps, float *orow, ew_f32x4 *copy = nullptr) {
     if constexpr (KIND == kNormRms) rms_norm_regs<R>(v, lane, n4, w, eps, orow, copy);
     else layer_norm_regs<R>(v, lane, n4, w, b, eps, orow, copy);
 }
+
+// A norm's weights in registers, loaded by a wave ahead of the row (lane l: float4 l + 64 i), and the norm
+// with them
+template <int KIND, int R>
+struct NormWeights {
+    ew_f32x4 w[R], b[KIND == kNormRms ? 1 : R];
+    __device__ __forceinline__ void load(int lane, int n4, const float *wp, const float *bp) {
+#pragma unroll
+        for (int i = 0; i < R; ++i)
+            if (lane + 64 * i < n4) {
+                w[i] = reinterpret_cast<const ew_f32x4 *>(wp)[lane + 64 * i];
+                if constexpr (KIND != kNormRms) b[i] = reinterpret_cast<const ew_f32x4 *>(bp)[lane + 64 * i];
+            }
+    }
+    __device__ __forceinline__ void norm(const ew_f32x4 (&v)[R], int lane, int n4, float eps, float *orow, ew_f32x4 *copy) const {
+        if constexpr (KIND == kNormRms) rms_norm_with<R>(v, lane, n4, [&](int i) { return w[i]; }, eps, orow, copy);
+        else layer_norm_with<R>(v, lane, n4, [&](int i) { return w[i]; }, [&](int i) { return b[i]; }, eps, orow, copy);
+    }
+};
 
 // ops.siluMul's element (src/ops.zig:429-439): gate / (1 + e^-gate) * up, rounded step by step in
 // that order (no contraction); e^x is the device's expf.
