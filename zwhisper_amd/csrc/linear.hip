@@ -290,7 +290,7 @@ struct Q8PartsOut {
 bool q8p_split_k(int64_t gx, int n_chunks, int nz = 1) {
     return gx < (nz > 1 ? ZWG_Q8P_SPLIT_BELOW_Z : ZWG_Q8P_SPLIT_BELOW) && n_chunks > 1;
 }
-// 32-row calls split x inside the stream kernel; 64-row ones too when k is split (small calls,
+// 32-row calls split x inside the kernel; 64-row ones too when k is split (small calls,
 // where the separate pass's launch costs more than the fused split), otherwise in a pass of their
 // own first.
 template <int MT>

@@ -248,7 +248,7 @@ __global__ __launch_bounds__(kQ8Threads) void linear_q8_stream_kernel(Q8Args a, 
     }
 }
 
-// Packed device weights (zwg_q8w): the same int8 and scales, laid out for the stream kernel so
+// Packed device weights (zwg_q8w): the same int8 and scales, laid out for the packed kernels so
 // that every wave-load is contiguous.  n is padded to whole slabs of 32 rows, k to whole chunks
 // of 256 (8 blocks); padding is zero (scale 0).
 //   q:      [slab][block][lane][16 bytes], lane l of (slab s, block b) holding
@@ -262,7 +262,7 @@ struct Q8Packed {
 };
 
 // Weight sets of one token-step launch over the same x (a decode step's q/k/v, or gate/up): set j
-// takes workgroups block_start[j] .. block_start[j + 1] - 1 of the stream kernel and elements
+// takes workgroups block_start[j] .. block_start[j + 1] - 1 of the packed kernel and elements
 // elem_start[j] .. elem_start[j + 1] - 1 of the split sum; all sets share x, k and the k split.
 constexpr int kQ8MaxGroup = 4;
 struct Q8Group {
@@ -279,7 +279,7 @@ struct Q8Group {
     float *part[kQ8MaxGroup]; // [n_split][m][n[j]] when the call is split
     // 1: a SwiGLU pair (count 2, n[0] == n[1]: the MLP's gate and up, src/llm.zig:207-210): each
     // workgroup takes the same columns of both sets and the call stores silu(gate) * up into
-    // out[0] (linear_q8p_stream_kernel; split calls through linear_split_sum_swiglu_kernel)
+    // out[0] (Q8pTile::store; split calls through linear_split_sum_swiglu_kernel)
     int32_t swiglu;
     // a SwiGLU pair of more than 32 rows: nullptr, or silu(gate) * up goes here split into f16 hi/lo
     // halves for the next 64-row-block call (linear_q8_xprep_kernel's layout; n % 128 == 0, so every
@@ -550,7 +550,7 @@ struct Q8pTile {
                 for (int g2 = 1; g2 < KB; ++g2) q += *reinterpret_cast<const f32x4 *>(at + g2 * NS * MS * OT);
                 v[j][p] = q + bv[j];
             }
-        const bool vec = n % 4 == 0; // rows 16-byte aligned
+        bool vec = n % 4 == 0; // rows 16-byte aligned (outputs start so; a group's partial sums may not)
         auto put = [&](float *o, f32x4 q) {
             if (vec) *reinterpret_cast<f32x4 *>(o) = q;
             else
@@ -561,6 +561,7 @@ struct Q8pTile {
 #pragma unroll
             for (int j = 0; j < NP; ++j) {
                 float *part = (PAIR ? grp.part[j] : GRP ? q8_pick(grp.part, set) : grp.part[0]) + (int64_t)split * m_all * n + o_at;
+                vec = n % 4 == 0 && (reinterpret_cast<uintptr_t>(part) & 15) == 0;
 #pragma unroll
                 for (int p = 0; p < PW; ++p)
                     if (o_r + 8 * p < m) put(part + (int64_t)8 * p * n, v[j][p]);
