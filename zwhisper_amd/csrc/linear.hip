@@ -350,6 +350,9 @@ hipError_t launch_q8p(const zwg_lin::Q8Args &a, const zwg_lin::Q8Group &g, const
         // more: 128 columns, half the x reads (32 x 8960 x 1536 in 18 splits 8.2, 64 columns 11.2)
         if (n_split > 1 && a.chunks_per_split == 1) return launch_q8p_tile<true, 1, 2, 1, 4>(a, g, xcvt, XS, n_split, nz, st);
         if (n_split > 1) return launch_q8p_tile<true, 1, 4, 1, 4>(a, g, xcvt, XS, n_split, nz, st);
+        // unsplit, at most half as many 128-column tiles as CUs: two waves per SIMD, each on half of every
+        // stage's blocks (a 32-row pair of 4864 x 896, 152 units: 10.8 -> 9.5, one row 10.4 -> 9.1)
+        if (units < 256) return launch_q8p_tile<false, 1, 4, 2, 4>(a, g, xcvt, XS, n_split, nz, st);
         // unsplit: 1 x 896 x 151936 31 (64 columns 42, 256 columns 38), 32 x 768 x 51864 16.0 (19, 15.4)
         return launch_q8p_tile<false, 1, 4, 1, 4>(a, g, xcvt, XS, n_split, nz, st);
     } else {
