@@ -1,0 +1,84 @@
+"""What the compiler made of the kernels' source, read from the built library's gfx950 code objects
+(on the CPU): properties that the results on one compiler's build cannot show."""
+from __future__ import annotations
+
+import os
+import re
+import struct
+import subprocess
+
+import pytest
+
+from zwhisper_amd import _lib
+
+LLVM = os.path.join(os.environ.get("ROCM_PATH", "/opt/rocm"), "llvm", "bin")
+
+
+def code_objects(path):
+    """The gfx950 code objects of the offload bundles in a library."""
+    data, magic, at, out = open(path, "rb").read(), b"__CLANG_OFFLOAD_BUNDLE__", 0, []
+    while (at := data.find(magic, at)) >= 0:
+        n, = struct.unpack_from("<Q", data, at + len(magic))
+        p = at + len(magic) + 8
+        for _ in range(n):
+            off, size, length = struct.unpack_from("<QQQ", data, p)
+            if size and data[p + 24:p + 24 + length].endswith(b"gfx950"):
+                out.append(data[at + off:at + off + size])
+            p += 24 + length
+        at += len(magic)
+    return out
+
+
+@pytest.fixture(scope="module")
+def objects(tmp_path_factory):
+    if not os.path.exists(os.path.join(LLVM, "llvm-objdump")):
+        pytest.skip("no ROCm LLVM tools")
+    files = []
+    for i, o in enumerate(code_objects(_lib.LIB_PATH)):
+        files.append(tmp_path_factory.mktemp("co") / f"{i}.co")
+        files[-1].write_bytes(o)
+    assert files, "no gfx950 code object in the library"
+    return files
+
+
+@pytest.fixture(scope="module")
+def packed_kernels(objects):
+    """{name: instructions} of the packed int8 kernels."""
+    kernels = {}
+    for f in objects:
+        if b"linear_q8p" not in f.read_bytes():
+            continue
+        text = subprocess.run([os.path.join(LLVM, "llvm-objdump"), "-d", "--mcpu=gfx950", str(f)], capture_output=True,
+                              text=True, check=True).stdout
+        body = None
+        for line in text.splitlines():
+            head = re.match(r"^[0-9a-f]+ <(.+)>:", line)
+            if head:
+                name = head.group(1)
+                body = kernels.setdefault(name, []) if "linear_q8p_short" in name or "linear_q8p_long" in name else None
+            elif body is not None and line.startswith("\t"):
+                body.append(line.split("//")[0].strip())
+    assert kernels
+    return kernels
+
+
+def is_copy(ins):
+    return ins.startswith("buffer_load") and ins.endswith(" lds")
+
+
+def test_copies_into_lds_are_issued_together(packed_kernels):
+    """A stage's copies into LDS are waited for by the count of the loads issued after them (s_waitcnt vmcnt,
+    in order), so no load into registers may be placed between them: each run of copies between two
+    barriers is unbroken."""
+    checked = 0
+    for name, body in packed_kernels.items():
+        seen, loads_since = False, 0
+        for ins in body:
+            if ins.startswith("s_barrier"):
+                seen, loads_since = False, 0
+            elif is_copy(ins):
+                assert not (seen and loads_since), f"{name}: a load between the copies of one stage"
+                seen, loads_since, checked = True, 0, checked + 1
+            elif ins.startswith(("buffer_load", "global_load")):
+                loads_since += 1
+    assert checked

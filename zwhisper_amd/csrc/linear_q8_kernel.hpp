@@ -486,6 +486,7 @@ struct Q8pTile {
         return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
                                              x_src, (int)x_lane, (int)(t < t_end && at < k ? (uint32_t)at * 4u : kOutOfRange), 0));
     }
+    // (the copies are waited for by the count of the loads after them, so none of those may move up)
     __device__ __forceinline__ void dma_x(int t, _Float16 *buf) const {
 #pragma unroll
         for (int u = 0; u < XL; ++u) {
@@ -493,6 +494,7 @@ struct Q8pTile {
             __builtin_amdgcn_raw_ptr_buffer_load_lds(x_src, (__attribute__((address_space(3))) void *)(buf + piece * 512), 16,
                                                      w_lane, t < t_end ? (uint32_t)((t * PIECES + piece) * 1024) : kOutOfRange, 0, 0);
         }
+        __builtin_amdgcn_sched_barrier(0);
     }
     __device__ __forceinline__ u32x4 load_w(int t, int b) const {
         const uint32_t at = (uint32_t)(t * SB + kg * NB + b) * 1024u;
