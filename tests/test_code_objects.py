@@ -82,3 +82,20 @@ def test_copies_into_lds_are_issued_together(packed_kernels):
             elif ins.startswith(("buffer_load", "global_load")):
                 loads_since += 1
     assert checked
+
+
+def test_copies_of_a_one_chunk_kernel_are_waited_for(packed_kernels):
+    """The short kernel's 64-row forms take at most two stages, both copied before the first barrier, with a
+    wait that leaves no copy in flight: nothing after it copies into LDS unwaited."""
+    checked = 0
+    for name, body in packed_kernels.items():
+        if "linear_q8p_short" not in name or not any(map(is_copy, body)):
+            continue
+        first = next(i for i, ins in enumerate(body) if ins.startswith("s_barrier"))
+        last = max(i for i, ins in enumerate(body) if is_copy(ins))
+        assert last < first, f"{name}: copies after the first barrier"
+        after = sum(ins.startswith(("buffer_load", "global_load")) for ins in body[last + 1:first])
+        waits = [int(m.group(1)) for ins in body[last:first] if (m := re.search(r"vmcnt\((\d+)\)", ins))]
+        assert waits and min(waits) <= after, f"{name}: {after} loads after the copies, waits {waits}"
+        checked += 1
+    assert checked

@@ -313,6 +313,7 @@ template <bool SHORT, int MT, int NS, int G, int SB>
 hipError_t launch_q8p_tile(const zwg_lin::Q8Args &a, zwg_lin::Q8Group g, const _Float16 *xcvt, bool XS, int n_split, int nz,
                            hipStream_t stream) {
     using namespace zwg_lin;
+    if (SHORT && MT == 2 && a.chunks_per_split != 1) return hipErrorInvalidValue; // its kernel has no loop
     const bool pair = g.swiglu != 0;
     int64_t gx = 0; // a SwiGLU pair's workgroups each take half their columns from both sets
     for (int j = 0; j < kQ8MaxGroup; ++j) {
@@ -357,8 +358,8 @@ hipError_t launch_q8p(const zwg_lin::Q8Args &a, const zwg_lin::Q8Group &g, const
         return launch_q8p_tile<false, 1, 4, 1, 4>(a, g, xcvt, XS, n_split, nz, st);
     } else {
         // one chunk per workgroup: 64 columns on four waves (64 x 1536 x 1536 in 6 splits 5.7, 128
-        // columns 6.6, the long kernel 6.9) while those, one per CU for their 96 KB of LDS, run at once
-        // (65 x 896 x 4864 in 4 splits, 608 of them: 19.6 with the split sum, the long kernel 14.5)
+        // columns 6.6, the long kernel 6.9) while those are at most one per CU (65 x 896 x 4864 in 4 splits,
+        // 608 of them, one at a time per CU: 19.6 with the split sum, the long kernel 14.5)
         if (n_split > 1 && a.chunks_per_split == 1 && 2 * units * n_split <= 256) return launch_q8p_tile<true, 2, 2, 2, 4>(a, g, xcvt, XS, n_split, nz, st);
         // more units than CUs, split: 256 columns (256 x 4864 x 896 in 10 splits 14.5, 128 columns
         // 16.1); fewer: 128 columns (64 x 8960 x 1536 in 18 splits 12.0, 256 columns 13.9)

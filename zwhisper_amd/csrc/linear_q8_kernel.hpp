@@ -610,11 +610,13 @@ struct Q8pTile {
 };
 
 // Short calls (a chunk or so of k per workgroup, about one workgroup per CU): nothing but the order
-// of a wave's own instructions hides latency.  Stages of 128 k, three LDS buffers: at stage t the
-// buffers of t and t + 1 are complete and t + 2's is being filled, so a call of one or two stages has
-// one barrier before its products and none after.  A stage is walked in units of one (block,
-// m-tile): while a unit's four MFMAs run, the wave reads the next unit's x operands, widens the next
-// block's weights, scales the previous unit's sums and (XS) splits its share of stage t + 2's x.
+// of a wave's own instructions hides latency.  Stages of 128 k.  32-row calls take any number of them
+// through three LDS buffers: at stage t the buffers of t and t + 1 are complete and t + 2's is being
+// filled, so a call of one or two stages has one barrier before its products and none after.  64-row
+// calls take one chunk, at most two stages (launch_q8p_tile refuses more), both loaded up front into
+// two buffers.  A stage is walked in units of one (block, m-tile): while a unit's four MFMAs run, the
+// wave reads the next unit's x operands, widens the next block's weights, scales the previous unit's
+// sums and splits its share of stage t + 2's x.
 // Left to the compiler, each operand was read directly before its MFMA.  Measured back to back with
 // weights from HBM, against one workgroup shape with a barrier per stage and 4-byte stores:
 // 32 x 768 x 768 in 3 splits 5.8 -> 4.6 us, 64 x 1536 x 1536 in 6 splits 9.1 -> 6.0 us, 256 x 896 x
@@ -623,25 +625,27 @@ template <int MT, int NS, int MS, bool XS, bool PAIR, bool GRP>
 __global__ __launch_bounds__(64 * NS * MS) __attribute__((amdgpu_waves_per_eu(2)))
 void linear_q8p_short_kernel(Q8Args a, Q8Group grp, const _Float16 *xcvt) {
     using Tile = Q8pTile<MT, NS, MS, 1, 4, XS, PAIR, GRP>;
-    constexpr int NB = 4, WT = Tile::WT, XQ = Tile::XQ, XL = Tile::XL, U = NB * WT;
-    constexpr int XS_BYTES = 3 * Tile::STAGE_HALVES * 2;
+    constexpr bool LOOP = MT == 1; // more than two stages
+    static_assert(XS || !LOOP, "the loop splits its own x");
+    constexpr int NB = 4, WT = Tile::WT, XQ = Tile::XQ, U = NB * WT, BUFS = LOOP ? 3 : 2;
+    constexpr int XS_BYTES = BUFS * Tile::STAGE_HALVES * 2;
     __shared__ __align__(16) char lds_all[XS_BYTES > Tile::OUT_BYTES ? XS_BYTES : Tile::OUT_BYTES];
-    auto &xs = *reinterpret_cast<_Float16(*)[3][Tile::STAGE_HALVES]>(lds_all);
+    auto &xs = *reinterpret_cast<_Float16(*)[BUFS][Tile::STAGE_HALVES]>(lds_all);
     const Tile w(a, grp, xcvt);
 
     f32x16 acc[WT];
 #pragma unroll
     for (int i = 0; i < WT; ++i) acc[i] = (f32x16){0};
     f32x4 xr[XQ];
-    u32x4 wq[3][NB];
-    typename Tile::Scales sc[3];
+    u32x4 wq[BUFS][NB];
+    typename Tile::Scales sc[BUFS];
 
     // stage t in buffer and register set `c`.  more: stages past t + 1 may follow (the last ones
     // load and put nothing)
     auto stage = [&](int t, auto c_c, auto more_c) {
         constexpr int c = decltype(c_c)::value, c2 = (c + 2) % 3;
         constexpr bool more = decltype(more_c)::value;
-        if constexpr (!XS && more) w.dma_x(t + 2, xs[c2]);
+        static_assert(LOOP || !more);
         half8 A[2][4]; // a unit's x operands
         half8 W[2][2]; // a block's widened weights
         f32x16 T[2];   // a unit's sums
@@ -667,7 +671,7 @@ void linear_q8p_short_kernel(Q8Args a, Q8Group grp, const _Float16 *xcvt) {
             if (u % WT == WT - 1 && u / WT + 1 < NB) widen(u / WT + 1);
             __builtin_amdgcn_sched_barrier(0);
             tt = __builtin_amdgcn_mfma_f32_32x32x16_f16(au[1], wu[0], tt, 0, 0, 0);
-            if (XS && more) { // a share of stage t + 2's x into LDS, its registers reloaded for t + 3
+            if constexpr (more) { // a share of stage t + 2's x into LDS, its registers reloaded for t + 3
 #pragma unroll
                 for (int e = u * XQ / U; e < (u + 1) * XQ / U; ++e) {
                     w.put_x(xs[c2], e, xr[e]);
@@ -684,16 +688,11 @@ void linear_q8p_short_kernel(Q8Args a, Q8Group grp, const _Float16 *xcvt) {
         scale(U - 1);
         if (more) sc[c] = w.load_s(t + 3);
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (more) {
-            // XS = false: the copies of stage t + 1 (issued a stage ago) are whole, those of t + 2 and the
-            // loads after them may still be in flight
-            if constexpr (!XS) __builtin_amdgcn_s_waitcnt(q8_vmcnt(XL + 2 * (NB + 1)));
-            __syncthreads();
-        }
+        if constexpr (more) __syncthreads();
         __builtin_amdgcn_sched_barrier(0);
     };
 
-    // first loads: x of stages 0 and 1, their weights and scales, then stage 2's
+    // first loads: x of stages 0 and 1, their weights and scales, then (LOOP) stage 2's
     f32x4 x0[XQ], x1[XQ];
     if constexpr (XS) {
 #pragma unroll
@@ -711,39 +710,43 @@ void linear_q8p_short_kernel(Q8Args a, Q8Group grp, const _Float16 *xcvt) {
         sc[c] = w.load_s(w.t_begin + c);
     }
     __builtin_amdgcn_sched_barrier(0);
-    if constexpr (XS) {
+    if constexpr (LOOP) {
 #pragma unroll
         for (int e = 0; e < XQ; ++e) xr[e] = w.load_x(w.t_begin + 2, e);
-    }
 #pragma unroll
-    for (int b = 0; b < NB; ++b) wq[2][b] = w.load_w(w.t_begin + 2, b);
-    sc[2] = w.load_s(w.t_begin + 2);
-    __builtin_amdgcn_sched_barrier(0);
+        for (int b = 0; b < NB; ++b) wq[2][b] = w.load_w(w.t_begin + 2, b);
+        sc[2] = w.load_s(w.t_begin + 2);
+        __builtin_amdgcn_sched_barrier(0);
+    }
     if constexpr (XS) {
 #pragma unroll
         for (int e = 0; e < XQ; ++e) w.put_x(xs[0], e, x0[e]);
 #pragma unroll
         for (int e = 0; e < XQ; ++e) w.put_x(xs[1], e, x1[e]);
     } else {
-        __builtin_amdgcn_s_waitcnt(q8_vmcnt(3 * (NB + 1)));
+        __builtin_amdgcn_s_waitcnt(q8_vmcnt(2 * (NB + 1)));
     }
     __syncthreads();
     __builtin_amdgcn_sched_barrier(0);
-    // turns of three stages, then the remaining one or two: the loop has no other way out, so the
-    // wait counts at its top are those of its own loads
     const int n_t = w.t_end - w.t_begin;
     int t = w.t_begin;
     constexpr std::integral_constant<int, 0> c0{};
     constexpr std::integral_constant<int, 1> c1{};
-    constexpr std::integral_constant<int, 2> c2{};
-    for (int p = n_t / 3; p > 0; --p, t += 3) {
-        stage(t, c0, std::true_type{});
-        stage(t + 1, c1, std::true_type{});
-        stage(t + 2, c2, std::true_type{});
+    if constexpr (LOOP) {
+        // turns of three stages, then the remaining one or two: the loop has no other way out, so the
+        // wait counts at its top are those of its own loads
+        constexpr std::integral_constant<int, 2> c2{};
+        for (int p = n_t / 3; p > 0; --p, t += 3) {
+            stage(t, c0, std::true_type{});
+            stage(t + 1, c1, std::true_type{});
+            stage(t + 2, c2, std::true_type{});
+        }
+        if (n_t % 3 > 0) stage(t, c0, std::false_type{});
+        if (n_t % 3 > 1) stage(t + 1, c1, std::false_type{});
+    } else {
+        stage(t, c0, std::false_type{});
+        if (n_t > 1) stage(t + 1, c1, std::false_type{});
     }
-    if (n_t % 3 > 0) stage(t, c0, std::false_type{});
-    if (n_t % 3 > 1) stage(t + 1, c1, std::false_type{});
-    if constexpr (!XS) __builtin_amdgcn_s_waitcnt(q8_vmcnt(0)); // the last, out-of-range copies into LDS
     __syncthreads();
     w.store(acc, reinterpret_cast<float *>(lds_all), grp);
 }
