@@ -99,3 +99,24 @@ def test_copies_of_a_one_chunk_kernel_are_waited_for(packed_kernels):
         assert waits and min(waits) <= after, f"{name}: {after} loads after the copies, waits {waits}"
         checked += 1
     assert checked
+
+
+def test_out_of_range_marker_is_in_the_checked_offset(packed_kernels):
+    """Loads past the last stage carry the offset 0x80000000, which the range check turns into zeros.  It
+    compares the lane's offset with the buffer's size less the scalar offset, which is undefined for a scalar
+    offset past the size: no load may have the marker as its scalar offset."""
+    checked = 0
+    for name, body in packed_kernels.items():
+        marked = set()
+        for ins in body:
+            op, _, rest = ins.partition(" ")
+            args = [a.strip() for a in rest.split(",")]
+            if op.startswith("buffer_load"):
+                scalar = args[2 if op.endswith("lds") or rest.endswith(" lds") else 3].split()[0]
+                assert scalar not in marked, f"{name}: {ins}"
+                checked += 1
+            elif op.startswith("s_") and args and re.fullmatch(r"s\d+", args[0]):
+                marked.discard(args[0])
+                if op in ("s_mov_b32", "s_cselect_b32") and "0x80000000" in args[1:]:
+                    marked.add(args[0])
+    assert checked

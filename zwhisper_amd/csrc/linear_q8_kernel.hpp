@@ -480,36 +480,44 @@ struct Q8pTile {
     }
 
     // the loads of stage t: x quad e (XS) or this wave's pieces into an LDS buffer, this wave's block
-    // b of its slab, and the stage's scales of this lane's row
+    // b of its slab, and the stage's scales of this lane's row.  A load past the last stage has its
+    // lane offset out of range (and scalar offset 0: the range check is against the size less that)
+    static __device__ __forceinline__ int lane_at(bool in, uint32_t at) { return (int)(in ? at : kOutOfRange); }
+    static __device__ __forceinline__ int scalar_at(bool in, uint32_t at) { return (int)(in ? at : 0u); }
     __device__ __forceinline__ f32x4 load_x(int t, int e) const {
         const int at = t * K + 16 * (x_g0 + e); // whole column groups: k % 32 == 0
-        return __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                             x_src, (int)x_lane, (int)(t < t_end && at < k ? (uint32_t)at * 4u : kOutOfRange), 0));
+        const bool in = t < t_end && at < k;
+        return __builtin_bit_cast(
+            f32x4, __builtin_amdgcn_raw_buffer_load_b128(x_src, lane_at(in, x_lane), scalar_at(in, (uint32_t)at * 4u), 0));
     }
     // (the copies are waited for by the count of the loads after them, so none of those may move up)
     __device__ __forceinline__ void dma_x(int t, _Float16 *buf) const {
+        const bool in = t < t_end;
 #pragma unroll
         for (int u = 0; u < XL; ++u) {
             const int piece = wave + NW * u;
             __builtin_amdgcn_raw_ptr_buffer_load_lds(x_src, (__attribute__((address_space(3))) void *)(buf + piece * 512), 16,
-                                                     w_lane, t < t_end ? (uint32_t)((t * PIECES + piece) * 1024) : kOutOfRange, 0, 0);
+                                                     lane_at(in, w_lane), scalar_at(in, (uint32_t)((t * PIECES + piece) * 1024)),
+                                                     0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
     }
     __device__ __forceinline__ u32x4 load_w(int t, int b) const {
+        const bool in = t < t_end;
         const uint32_t at = (uint32_t)(t * SB + kg * NB + b) * 1024u;
         return __builtin_bit_cast(
-            u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_src, (int)w_lane, (int)(t < t_end ? at : kOutOfRange), POLICY));
+            u32x4, __builtin_amdgcn_raw_buffer_load_b128(q_src, lane_at(in, w_lane), scalar_at(in, at), POLICY));
     }
     __device__ __forceinline__ Scales load_s(int t) const {
+        const bool in = t < t_end;
         const uint32_t at = (uint32_t)(t / SPC) * (32u * kQ8ChunkBlocks * 4u) + 4u * (uint32_t)(t % SPC * SB + kg * NB);
-        const int so = (int)(t < t_end ? at : kOutOfRange);
+        const int lo = lane_at(in, s_lane), so = scalar_at(in, at);
         if constexpr (NB == 4)
-            return __builtin_bit_cast(Scales, __builtin_amdgcn_raw_buffer_load_b128(s_src, (int)s_lane, so, POLICY));
+            return __builtin_bit_cast(Scales, __builtin_amdgcn_raw_buffer_load_b128(s_src, lo, so, POLICY));
         else if constexpr (NB == 2)
-            return __builtin_bit_cast(Scales, __builtin_amdgcn_raw_buffer_load_b64(s_src, (int)s_lane, so, POLICY));
+            return __builtin_bit_cast(Scales, __builtin_amdgcn_raw_buffer_load_b64(s_src, lo, so, POLICY));
         else
-            return __builtin_bit_cast(Scales, __builtin_amdgcn_raw_buffer_load_b32(s_src, (int)s_lane, so, POLICY));
+            return __builtin_bit_cast(Scales, __builtin_amdgcn_raw_buffer_load_b32(s_src, lo, so, POLICY));
     }
     // XS: quad e split into an LDS buffer (a quad is half of one lane's 8-element piece)
     __device__ __forceinline__ void put_x(_Float16 *buf, int e, const f32x4 &v) const {
@@ -761,8 +769,11 @@ void linear_q8p_short_kernel(Q8Args a, Q8Group grp, const _Float16 *xcvt) {
 // 128 k stages with a barrier, an LDS round trip per operand and 4-byte stores: the 64-row
 // logits of 151936 x 1536 91 -> 79 us, a 256-row SwiGLU pair of 4864 x 896 37 -> 20 us, the one-row
 // logits of 151936 x 896 58 -> 31 us, 1001 x 1536 x 8960 (the tiled kernel before) 120 -> 71 us.
+// The 64 x 128 tile is held to three workgroups per CU; its registers would allow four, which measured
+// slower (1001 x 1536 x 8960 75.3 us for 73.6, the 64-row logits 88.6 for 86.9).
 template <int MT, int NS, int KB, int SB, bool XS, bool PAIR, bool GRP>
-__global__ __launch_bounds__(64 * NS * KB) __attribute__((amdgpu_waves_per_eu(SB == 2 ? 3 : 2)))
+__global__ __launch_bounds__(64 * NS * KB) __attribute__((amdgpu_waves_per_eu(
+    SB == 2 ? 3 : MT == 1 && KB == 1 ? 4 : 2, SB == 2 && NS == 4 ? 3 : 8)))
 void linear_q8p_long_kernel(Q8Args a, Q8Group grp, const _Float16 *xcvt) {
     using Tile = Q8pTile<MT, NS, 1, KB, SB, XS, PAIR, GRP>;
     constexpr int WT = Tile::WT, XQ = Tile::XQ, NB = Tile::NB;
