@@ -120,3 +120,20 @@ def test_out_of_range_marker_is_in_the_checked_offset(packed_kernels):
                 if op in ("s_mov_b32", "s_cselect_b32") and "0x80000000" in args[1:]:
                     marked.add(args[0])
     assert checked
+
+
+def test_row_kernels_do_not_spill(objects):
+    """The split sum + residual + norm kernel (a thread per float4 column, up to 1024 of them: 128 VGPRs each)
+    keeps its registers at every row width, with four waves per SIMD."""
+    checked = 0
+    for f in objects:
+        notes = subprocess.run([os.path.join(LLVM, "llvm-readelf"), "--notes", str(f)], capture_output=True, text=True,
+                               check=True).stdout
+        for kernel in notes.split(".args:")[1:]:
+            name = re.search(r"\.name: +(_Z\S+)", kernel)
+            if not name or "linear_split_sum_add_ln_wide" not in name.group(1):
+                continue
+            values = {k: int(v) for k, v in re.findall(r"\.(\w+): +(\d+)", kernel)}
+            assert values["vgpr_spill_count"] == 0 and values["vgpr_count"] <= 128, (name.group(1), values)
+            checked += 1
+    assert checked >= 24  # two norms, twelve row widths

@@ -189,6 +189,31 @@ def test_step_bit_exact_with_composed_calls(torch, ctx, ns, H):
                     assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]), (step, li, s)
 
 
+@pytest.mark.parametrize("ns", [1792, 2048])
+def test_step_bit_exact_wide_rows(torch, ctx, ns):
+    """The widest states: the split sum + residual + layer norm kernel with seven and eight waves per row."""
+    import zwhisper_amd as z
+
+    rng = np.random.default_rng(ns)
+    H, n_vocab, n_tctx, n_actx, m = ns // 128, 300, 16, 40, 3
+    print(f"decoder step n_state={ns} heads={H} windows {m}", flush=True)
+    mdl = model(rng, ns, 1, n_vocab, n_tctx)
+    with contextlib.ExitStack() as st:
+        dec = st.enter_context(make_decoder(z, ctx, mdl, H, n_tctx, n_actx, m))
+        comp = Composed(torch, ctx, dec, H, m)
+        st.callback(comp.close)
+        enc = torch.from_numpy(rng.standard_normal((m, n_actx, ns)).astype(np.float32)).cuda()
+        dec.set_audio(enc, m, 0)
+        comp.set_audio(enc, m, 0)
+        la, lb = torch.empty(m, n_vocab, device="cuda"), torch.empty(m, n_vocab, device="cuda")
+        pos = np.array([0, 3, 15], np.int32)
+        tok = rng.integers(0, n_vocab, m).astype(np.int32)
+        dec.step(torch.from_numpy(tok).cuda(), torch.from_numpy(pos).cuda(), la, 0)
+        comp.step(mdl["te"], mdl["pe"], tok, pos, 0, lb)
+        torch.cuda.synchronize()
+        assert bool(torch.isfinite(la).all()) and torch.equal(la, lb)
+
+
 def test_step_against_oracle(torch, ctx):
     import oracle
     import zwhisper_amd as z

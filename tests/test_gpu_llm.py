@@ -211,6 +211,30 @@ def test_step_bit_exact_33_to_64_rows(torch, ctx, m):
                     assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]), (step, li, s)
 
 
+@pytest.mark.parametrize("m", [3, 40])
+@pytest.mark.parametrize("ne", [1920, 2304, 2560, 3584, 4096])
+def test_step_bit_exact_wide_rows(torch, ctx, ne, m):
+    """Rows of more than 2048 floats: the split sum + residual + norm kernel's widest forms (the norm's weights
+    handed to the first wave through LDS), 40 rows with the normalised row split for the next call."""
+    import zwhisper_amd as z
+    from zwhisper_amd import _lib
+
+    rng = np.random.default_rng(ne + m)
+    H, Hk, nff, n_vocab, n_ctx = ne // 128, 1, 512, 300, 16
+    print(f"llm step n_embd={ne} heads {H}/{Hk} n_ff={nff} sequences {m}", flush=True)
+    mdl = model(rng, ne, H, Hk, nff, 1, n_vocab)
+    with contextlib.ExitStack() as st:
+        lm = st.enter_context(make_llm(z, ctx, mdl, H, Hk, nff, n_ctx, m))
+        kv = st.enter_context(z.KVCache(ctx, 1, m, n_ctx, Hk, 128, _lib.KV_KT, 1e6))
+        la, lb = torch.empty(m, n_vocab, device="cuda"), torch.empty(m, n_vocab, device="cuda")
+        pos = rng.integers(0, n_ctx, m).astype(np.int32)
+        tok = rng.integers(0, n_vocab, m).astype(np.int32)
+        lm.step(torch.from_numpy(tok).cuda(), torch.from_numpy(pos).cuda(), la, 0)
+        composed_step(torch, ctx, lm, kv, mdl["embd"], H, Hk, tok, pos, 0, lb)
+        torch.cuda.synchronize()
+        assert bool(torch.isfinite(la).all()) and torch.equal(la, lb)
+
+
 def test_step_against_oracle(torch, ctx):
     import oracle
     import zwhisper_amd as z

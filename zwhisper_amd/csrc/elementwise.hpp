@@ -57,7 +57,7 @@ __device__ __forceinline__ float wave_sum(float v) {
 // differs from the reference's 16-lane vector order (a few f32 ulps).  Every kernel that normalises
 // a row goes through this function, so a fused norm equals the separate one bit for bit.
 // copy: nullptr, or a second destination of the output float4s (same index as in orow).
-// The norm weights (w, b: callables of i) may be loaded before the row is whole.
+// w, b: callables of i, the norm's weights of float4 lane + 64 i (from memory, or loaded ahead of the row).
 template <int R, typename W, typename B>
 __device__ __forceinline__ void layer_norm_with(const ew_f32x4 (&v)[R], int lane, int n4, W w, B b, float eps, float *orow,
                                                 ew_f32x4 *copy) {
@@ -148,25 +148,6 @@ __device__ __forceinline__ void norm_regs(const ew_f32x4 (&v)[R], int lane, int 
     if constexpr (KIND == kNormRms) rms_norm_regs<R>(v, lane, n4, w, eps, orow, copy);
     else layer_norm_regs<R>(v, lane, n4, w, b, eps, orow, copy);
 }
-
-// A norm's weights in registers, loaded by a wave ahead of the row (lane l: float4 l + 64 i), and the norm
-// with them
-template <int KIND, int R>
-struct NormWeights {
-    ew_f32x4 w[R], b[KIND == kNormRms ? 1 : R];
-    __device__ __forceinline__ void load(int lane, int n4, const float *wp, const float *bp) {
-#pragma unroll
-        for (int i = 0; i < R; ++i)
-            if (lane + 64 * i < n4) {
-                w[i] = reinterpret_cast<const ew_f32x4 *>(wp)[lane + 64 * i];
-                if constexpr (KIND != kNormRms) b[i] = reinterpret_cast<const ew_f32x4 *>(bp)[lane + 64 * i];
-            }
-    }
-    __device__ __forceinline__ void norm(const ew_f32x4 (&v)[R], int lane, int n4, float eps, float *orow, ew_f32x4 *copy) const {
-        if constexpr (KIND == kNormRms) rms_norm_with<R>(v, lane, n4, [&](int i) { return w[i]; }, eps, orow, copy);
-        else layer_norm_with<R>(v, lane, n4, [&](int i) { return w[i]; }, [&](int i) { return b[i]; }, eps, orow, copy);
-    }
-};
 
 // ops.siluMul's element (src/ops.zig:429-439): gate / (1 + e^-gate) * up, rounded step by step in
 // that order (no contraction); e^x is the device's expf.

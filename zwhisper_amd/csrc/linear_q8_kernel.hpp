@@ -1164,7 +1164,8 @@ __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(co
 #pragma clang fp contract(off)
     typedef float f4 __attribute__((ext_vector_type(4)));
     constexpr int B = 24;
-    __shared__ f4 rowbuf[64 * R];
+    constexpr bool kLayerNorm = NORM != zwg_ew::kNormRms;
+    __shared__ f4 rowbuf[64 * R], wbuf[64 * R], bbuf[kLayerNorm ? 64 * R : 1];
     const int c = threadIdx.x; // this thread's float4 column
     const int row = (int)blockIdx.x;
     if (row >= m) return;
@@ -1178,10 +1179,15 @@ __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(co
         xo = xr[c];
         if (bias) bo = reinterpret_cast<const f4 *>(bias)[c];
     }
-    // the first wave's norm weights, in flight with the partials rather than a round trip behind them (the
-    // small.en decoder step 1460 -> 1436 us over its 36 launches)
-    zwg_ew::NormWeights<NORM, R> nw;
-    if (c < 64) nw.load(c, n4, r.ln_w, r.ln_b);
+    // the norm's weights, each thread its column's, in flight with the partials rather than a round trip
+    // behind them (the small.en decoder step 1460 -> 1436 us over its 36 launches), and to the first wave
+    // through LDS: held in its registers they cost every wave as many, and spilled at R = 14 and 16 (64 rows of
+    // 4096 floats, a step of eight layers: 939 us loaded after the sums, 961 so, 771 through LDS)
+    f4 nw = {0.f, 0.f, 0.f, 0.f}, nb = {0.f, 0.f, 0.f, 0.f};
+    if (live) {
+        nw = reinterpret_cast<const f4 *>(r.ln_w)[c];
+        if constexpr (kLayerNorm) nb = reinterpret_cast<const f4 *>(r.ln_b)[c];
+    }
     f4 s = {0.f, 0.f, 0.f, 0.f};
     for (int q0 = 0; q0 < n_split; q0 += B) {
         f4 t[B];
@@ -1200,13 +1206,21 @@ __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(co
         xr[c] = nx;
     }
     rowbuf[c] = nx;
+    wbuf[c] = nw;
+    if constexpr (kLayerNorm) bbuf[c] = nb;
     __syncthreads();
     if (c < 64) {
         zwg_ew::ew_f32x4 v[R];
 #pragma unroll
         for (int i = 0; i < R; ++i) v[i] = rowbuf[c + 64 * i];
         // with xcvt the normalised row also goes back into rowbuf (past n4 it stays zero)
-        nw.norm(v, c, n4, r.eps, r.ln_out + (int64_t)row * n, r.xcvt ? rowbuf : nullptr);
+        float *const orow = r.ln_out + (int64_t)row * n;
+        f4 *const copy = r.xcvt ? rowbuf : nullptr;
+        const auto w = [&](int i) { return wbuf[c + 64 * i]; };
+        if constexpr (kLayerNorm)
+            zwg_ew::layer_norm_with<R>(v, c, n4, w, [&](int i) { return bbuf[c + 64 * i]; }, r.eps, orow, copy);
+        else
+            zwg_ew::rms_norm_with<R>(v, c, n4, w, r.eps, orow, copy);
     }
     if (r.xcvt) {
         __syncthreads();
