@@ -421,7 +421,8 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
             // store to out it cannot tell apart) would wait one memory round trip each.  The loads
             // go through a descriptor ending at the tile's last element (rows past m read 0), with
             // the lane's part of the offset in one VGPR and the register's row in the SGPR part.
-            const __amdgpu_buffer_rsrc_t o_src = rsrc(a.out + (int64_t)m0 * a.ldo + n0, (uint32_t)(span * 4));
+            char *const o_tile = reinterpret_cast<char *>(a.out + (int64_t)m0 * a.ldo + n0);
+            const __amdgpu_buffer_rsrc_t o_src = rsrc(reinterpret_cast<const float *>(o_tile), (uint32_t)(span * 4));
             const int ld4 = (int)a.ldo * 4;
             const int vo = (wm * WM + 4 * (lane >> 5)) * ld4 + (wn * WN + r32) * 4;
 #pragma unroll
@@ -443,7 +444,8 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
                     for (int r = 0; r < 16; ++r) {
                         const int row = m0 + wm * WM + i * 32 + 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
                         if (row >= a.m) continue;
-                        a.out[(int64_t)row * a.ldo + col] = res[j][r] + (acc[i][j][r] + bj);
+                        const uint32_t at = (uint32_t)vo + (uint32_t)((i * 32 + 8 * (r >> 2) + (r & 3)) * ld4 + j * 128);
+                        *reinterpret_cast<float *>(o_tile + at) = res[j][r] + (acc[i][j][r] + bj);
                     }
                 }
             }
@@ -476,8 +478,8 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
     }
 }
 
-// The f16 64 x 256 tile is held to 80 VGPRs, three 8-wave workgroups per CU (its epilogue's residual
-// rows would take it to 82, two workgroups: 6000 x 384 x 1536 28.7 -> 33.2 us).
+// The f16 64 x 256 tile is held to 80 VGPRs (it fits them without a spill), three 8-wave workgroups per
+// CU: its epilogue's residual rows would take it to 82, two workgroups (6000 x 384 x 1536 28.7 -> 33.2 us).
 template <int BM, int BN, int WMODE, int NWN = 2, bool KSPLIT = false>
 __global__ __launch_bounds__(128 * NWN) __attribute__((amdgpu_waves_per_eu(WMODE == kWF16 && BM == 64 && BN == 256 ? 6 : 1)))
 void linear_mfma_kernel(LinearArgs a) {

@@ -1181,8 +1181,8 @@ __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(co
     }
     // the norm's weights, each thread its column's, in flight with the partials rather than a round trip
     // behind them (the small.en decoder step 1460 -> 1436 us over its 36 launches), and to the first wave
-    // through LDS: held in its registers they cost every wave as many, and spilled at R = 14 and 16 (64 rows of
-    // 4096 floats, a step of eight layers: 939 us loaded after the sums, 961 so, 771 through LDS)
+    // through LDS: held in its registers they cost every wave as many, and spilled from R = 14 on (a step
+    // of eight layers of 4096 floats, 64 rows: 961 us so, 771 through LDS)
     f4 nw = {0.f, 0.f, 0.f, 0.f}, nb = {0.f, 0.f, 0.f, 0.f};
     if (live) {
         nw = reinterpret_cast<const f4 *>(r.ln_w)[c];
