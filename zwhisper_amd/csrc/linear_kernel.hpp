@@ -100,6 +100,13 @@ __device__ __forceinline__ half8 int8x8_to_half8(uint32_t w0, uint32_t w1) {
     return r;
 }
 
+// LDS values passed between the lanes of one wave: the hardware keeps the wave's accesses in order, and
+// this keeps the compiler's.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc(const void *base, uint32_t bytes) {
     return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(base), 0, (int)bytes, 0x00020000);
 }
@@ -344,10 +351,11 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
         }
     }
     // Rows of the output whose 16-byte groups are aligned go out 16 bytes per lane: each wave passes its
-    // 32 x 32 blocks through its own LDS tile (rows of 36 floats; a wave's LDS accesses stay in order,
-    // so no barrier) and stores 8 rows of 128 bytes at a time.  A 4-byte store costs the address unit
-    // as many cycles as a 16-byte one: 24000 x 512 x 2048 with GELU 136 -> 124 us, 1000 x 512 x 512
-    // with the residual add 10.1 -> 8.1, the other encoder shapes 1.01 to 1.3 times as fast.
+    // accumulators, 32 / TN rows of WN columns at a time, through its own LDS tile (rows of WN + 4 floats; a
+    // wave's LDS accesses stay in order, so fences for the compiler and no barrier) and stores whole row
+    // pieces.  A 4-byte store costs the address unit as many cycles as a 16-byte one: 24000 x 512 x 2048
+    // with GELU 136 -> 124 us, 1000 x 512 x 512 with the residual add 10.1 -> 8.1, the other encoder shapes
+    // 1.01 to 1.3 times as fast.
     constexpr int kLd = WN + 4, kCh = 32 / TN; // floats per tile row; rows of a chunk
     constexpr int kLpr = WN / 4, kRpp = 64 / kLpr, kP = kCh / kRpp; // lanes per row, rows per piece, pieces
     static_assert(TN == 1 || TN == 2, "a chunk's rows are whole register quads");
@@ -394,6 +402,7 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
 #pragma unroll
                     for (int r = 0; r < 16 / TN; ++r)
                         tile[(8 * (r >> 2) + 4 * (lane >> 5) + (r & 3)) * kLd + j * 32 + r32] = acc[i][j][h * (16 / TN) + r] + bj[j];
+                wave_lds_fence(); // the rows to the lanes that store them
 #pragma unroll
                 for (int p = 0; p < kP; ++p) {
                     f32x4 v = *reinterpret_cast<const f32x4 *>(tile + (t_r + kRpp * p) * kLd + t_c);
@@ -408,6 +417,7 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
                         __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4_st, v), o_dst, (int)((row * ldd + col0) * 4),
                                                                0, kNonTemporal);
                 }
+                wave_lds_fence(); // every lane has its piece before the next chunk's writes
             }
         }
         return;
