@@ -10,10 +10,10 @@
 //     Q = q(A); k(A), v(A) -> self cache rows at pos  stream + linear_split_sum_qkv_kernel, which
 //                                                     also writes the key counts pos + 1
 //     T = attention(Q, self cache[0 .. pos])           decode kernel (+ merge)
-//     X += o(T); A = cross_ln(X)                       stream + linear_split_sum_add_ln_kernel
+//     X += o(T); A = cross_ln(X)                       stream + linear_split_sum_add_ln_wide_kernel
 //     T = attention(cq(A), cross cache)                stream (partials to P) + decode kernel, whose
 //                                                     q load adds the partials and bias (+ merge)
-//     X += co(T); A = mlp_ln(X)                        stream + linear_split_sum_add_ln_kernel
+//     X += co(T); A = mlp_ln(X)                        stream + linear_split_sum_add_ln_wide_kernel
 //     H = gelu(mlp0(A))                                stream + split sum (GELU in its store)
 //     X += mlp1(H); A = next layer's attn_ln(X), or the final ln after the last layer
 //   logits = A . te^T                                  stream (unsplit)

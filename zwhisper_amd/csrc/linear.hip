@@ -210,8 +210,8 @@ constexpr int q8p_unit() { return MT == 1 ? 64 : 128; }
 #define ZWG_Q8P_FUSED_ROWS 256
 
 
-// Row kernels of n <= 2048 floats (a wave per row, n / 256 float4 per lane, rounded up), one
-// wave per workgroup: a decode step's few rows then read their partials through as many CUs as
+// Row kernels of n <= 4096 floats (a wave per row, n / 256 float4 per lane, rounded up, or a thread per
+// float4), one row per workgroup: a decode step's few rows then read their partials through as many CUs as
 // there are rows (four rows per workgroup put a 32-row step's 1.3 MB of partial loads through 8
 // CUs' load paths)
 constexpr int kMaxRowN = 4096; // the row kernels' widest row: 16 float4 per lane
@@ -237,27 +237,12 @@ hipError_t launch_rows(int32_t n, int32_t m, hipStream_t stream, Args... args) {
     return hipGetLastError();
 }
 template <int R, int NORM>
-struct AddLnRows {
-    static void launch(dim3 g, dim3 b, hipStream_t st, const float *part, const float *bias, zwg_lin::Q8ResLn r,
-                       int32_t m, int32_t n, int32_t n_split) {
-        zwg_lin::linear_split_sum_add_ln_kernel<R, NORM><<<g, b, 0, st>>>(part, bias, r, m, n, n_split);
-    }
-};
-template <int R, int NORM>
 struct AddLnWideRows { // R waves per row: the block size is the kernel's own
     static void launch(dim3 g, dim3, hipStream_t st, const float *part, const float *bias, zwg_lin::Q8ResLn r,
                        int32_t m, int32_t n, int32_t n_split) {
         zwg_lin::linear_split_sum_add_ln_wide_kernel<R, NORM><<<g, dim3(64 * R), 0, st>>>(part, bias, r, m, n, n_split);
     }
 };
-// the split sum + residual + norm kernel: one thread per float4 column (1) or one wave per row (0).
-// Paired runs on one box, per step: Whisper small.en decoder (32 windows) 1563 -> 1537 us, Qwen2.5-1.5B
-// decode (64 sequences; its down projection's sums take 35 splits) 4394 -> 4198 us.
-#ifndef ZWG_ADDLN_WIDE
-#define ZWG_ADDLN_WIDE 1
-#endif
-template <int R, int NORM>
-using AddLnChosen = std::conditional_t<ZWG_ADDLN_WIDE != 0, AddLnWideRows<R, NORM>, AddLnRows<R, NORM>>;
 template <int R, int NORM>
 struct EmbedLnRows {
     static void launch(dim3 g, dim3 b, hipStream_t st, zwg_lin::Q8Packed te, int32_t n_vocab, const int32_t *tok,
@@ -269,8 +254,8 @@ struct EmbedLnRows {
 
 // kvs (a q/k/v group, sets 0, 1, 2): the split sum stores into q_out and the KV cache
 // (linear_split_sum_qkv_kernel), so the call is always split, in two at least.  resln (one set,
-// n <= 2048): the split sum adds into the residual stream and normalises the rows
-// (linear_split_sum_add_ln_kernel), likewise always split.
+// n <= kMaxRowN): the split sum adds into the residual stream and normalises the rows
+// (linear_split_sum_add_ln_wide_kernel), likewise always split.
 // po (one set): the partials go to po->part (at most po->max_parts splits, at least two) and no
 // split sum is launched; the split count is returned in po->n_split.
 struct Q8PartsOut {
@@ -457,9 +442,9 @@ int run_q8p_group(zwg_ctx *ctx, const zwg_lin::Q8Args &base, zwg_lin::Q8Group g,
         // the caller adds the partials (attention's q load)
     } else if (resln) {
         e = resln->norm == zwg_ew::kNormRms
-                ? launch_rows<AddLnChosen, zwg_ew::kNormRms>(g.n[0], a.m, ctx->stream, (const float *)g.part[0],
+                ? launch_rows<AddLnWideRows, zwg_ew::kNormRms>(g.n[0], a.m, ctx->stream, (const float *)g.part[0],
                                                              g.bias[0], *resln, a.m, g.n[0], n_split)
-                : launch_rows<AddLnChosen, zwg_ew::kNormLayer>(g.n[0], a.m, ctx->stream, (const float *)g.part[0],
+                : launch_rows<AddLnWideRows, zwg_ew::kNormLayer>(g.n[0], a.m, ctx->stream, (const float *)g.part[0],
                                                                g.bias[0], *resln, a.m, g.n[0], n_split);
         if (e != hipSuccess) return fail_hip(ctx, "split-sum + residual + norm kernel launch", e);
     } else if (n_split > 1 && pair) {
@@ -761,7 +746,7 @@ int zwg_host::linear_q8w_qkv_kv(zwg_ctx *ctx, const float *x, uint64_t m, const 
 
 // x += xin . W^T + bias and ln_out = the norm of x (layer norm with ln_w, ln_b, or RMS norm with
 // ln_w; eps) for a decode step's or a prompt batch's rows (m <= 256, n <= 4096): one stream launch and
-// linear_split_sum_add_ln_kernel; a call too short to split k (k <= 256) runs the add epilogue and
+// linear_split_sum_add_ln_wide_kernel; a call too short to split k (k <= 256) runs the add epilogue and
 // the norm as two launches, with the same results.  xcvt_out (more than 32 rows): ln_out also split
 // for the next call (q8w_xcvt_halves(m, n) halves), which takes it as xcvt_in.
 int zwg_host::linear_q8w_add_ln(zwg_ctx *ctx, const float *xin, uint64_t m, const zwg_q8w *w, const float *bias,

@@ -1076,9 +1076,13 @@ __global__ __launch_bounds__(256) void linear_split_sum_qkv_kernel(Q8Group grp, 
 // of x += sum over splits (in split order) of part[s][i] + bias -- as
 // linear_split_sum_group_kernel with the add epilogue forms it -- then ln_out[i] = the norm of
 // x[i] (NORM: zwg_ew::kNormLayer or kNormRms, through the functions layer_norm_kernel and
-// rms_norm_kernel use).  So x and ln_out equal the split sum and the norm launch bit for bit.  One wave per row of n <= 256 R floats; the
-// residual row, the bias and the partials of B splits at a time are loaded before any add.  One
-// one-wave workgroup per row.
+// rms_norm_kernel use).  So x and ln_out equal the split sum and the norm launch bit for bit.  One thread
+// per float4 column (R waves per row, n <= 256 R floats), with up to 24 of its column's splits in flight
+// at once: with a wave per row instead, each lane walked R columns in batches of 48 / R splits (the
+// Qwen2.5-1.5B down projection's 35 splits of 1536-float rows: 18 batches of loads one after another;
+// per step, paired: Whisper small.en decoder over 32 windows 1563 us so, 1537 with a thread per column,
+// Qwen2.5-1.5B decode over 64 sequences 4394 and 4198).  The new row goes through LDS to the first wave,
+// which normalises it.
 struct Q8ResLn {
     float *x; // [m][n] residual stream, updated in place
     const float *ln_w, *ln_b; // ln_b unused by the RMS norm
@@ -1086,77 +1090,10 @@ struct Q8ResLn {
     float eps;
     int32_t norm; // zwg_ew::kNormLayer or kNormRms (host side: which instantiation)
     // nullptr, or the normalised rows also split into f16 hi/lo halves for the next call of 64-row blocks
-    // (linear_q8_xprep_kernel's layout and values, the last block's rows past m zero); the one-thread-per-column
-    // kernel only
+    // (linear_q8_xprep_kernel's layout and values, the last block's rows past m zero)
     _Float16 *xcvt;
 };
 
-template <int R, int NORM>
-__global__ __launch_bounds__(64) void linear_split_sum_add_ln_kernel(const float *part, const float *bias, Q8ResLn r,
-                                                                     int32_t m, int32_t n, int32_t n_split) {
-#pragma clang fp contract(off)
-    typedef float f4 __attribute__((ext_vector_type(4)));
-    constexpr int B = 48 / R < 16 ? 48 / R : 16; // splits whose loads go out together (B R float4 per lane)
-    const int lane = threadIdx.x;
-    const int row = (int)blockIdx.x; // one wave per workgroup, one row per wave
-    if (row >= m) return;
-    const int n4 = n >> 2;
-    const int64_t step = (int64_t)m * n4; // float4s of one split
-    const f4 *p = reinterpret_cast<const f4 *>(part) + (int64_t)row * n4;
-    // the residual row and the bias first: their loads share the partials' round trip
-    f4 *xr = reinterpret_cast<f4 *>(r.x + (int64_t)row * n);
-    f4 xo[R], bo[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-        const int c = lane + 64 * i;
-        if (c < n4) {
-            xo[i] = xr[c];
-            bo[i] = bias ? reinterpret_cast<const f4 *>(bias)[c] : (f4){0.f, 0.f, 0.f, 0.f};
-        }
-    }
-    f4 s[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) s[i] = (f4){0.f, 0.f, 0.f, 0.f};
-    for (int q0 = 0; q0 < n_split; q0 += B) {
-        f4 t[B][R];
-#pragma unroll
-        for (int j = 0; j < B; ++j)
-#pragma unroll
-            for (int i = 0; i < R; ++i) {
-                const int c = lane + 64 * i;
-                if (q0 + j < n_split && c < n4) t[j][i] = p[(q0 + j) * step + c];
-            }
-#pragma unroll
-        for (int j = 0; j < B; ++j)
-#pragma unroll
-            for (int i = 0; i < R; ++i) {
-                const int c = lane + 64 * i;
-                if (q0 + j < n_split && c < n4) s[i] = q0 + j == 0 ? t[j][i] : s[i] + t[j][i];
-            }
-    }
-    zwg_ew::ew_f32x4 v[R];
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-        const int c = lane + 64 * i;
-        if (c < n4) {
-            f4 val = s[i];
-            if (bias) val = val + bo[i];
-            const f4 nx = xo[i] + val;
-            xr[c] = nx;
-            v[i] = nx;
-        } else {
-            v[i] = (zwg_ew::ew_f32x4){0.f, 0.f, 0.f, 0.f};
-        }
-    }
-    zwg_ew::norm_regs<NORM, R>(v, lane, n4, r.ln_w, r.ln_b, r.eps, r.ln_out + (int64_t)row * n);
-}
-
-// The same sums, residual add and norm with one thread per float4 column (R waves per row, n <=
-// 256 R floats): each thread has up to 24 of its column's splits in flight at once, where the
-// one-wave kernel walks R columns per lane in batches of 48 / R splits (the Qwen2.5-1.5B down
-// projection's 35 splits of 1536-float rows: 18 batches of loads one after another per wave).
-// The new row goes through LDS to the first wave, which normalises it with norm_regs exactly as
-// the one-wave kernel does (so the two give the same bits).
 template <int R, int NORM>
 __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(const float *part, const float *bias,
                                                                               Q8ResLn r, int32_t m, int32_t n,
