@@ -51,7 +51,7 @@ int zwg_encoder_layer_dev(zwg_ctx *ctx, float *x, uint64_t n_windows, uint64_t n
     if (ctx->dense_math == ZWG_DENSE_X3 && (d == 64 || d == 128) && n_ctx % 4 == 0 &&
         2 * rows * ns + 2 * img_floats <= zwg_encoder_layer_scratch(rows, ns)) {
         float *Q = B, *Kimg = Q + rows * ns, *Vimg = Kimg + img_floats;
-        if ((rc = zwg_linear_epi_dev(ctx, A, rows, ns, w->q_w, ZWG_W_F16, w->q_b, ns, Q, ns, ZWG_EPI_NONE)) != ZWG_OK)
+        if ((rc = linear_f16_keep(ctx, A, rows, ns, w->q_w, w->q_b, ns, Q, ns, ZWG_EPI_NONE)) != ZWG_OK)
             return rc;
         if ((rc = linear_f16_image(ctx, A, rows, ns, w->k_w, nullptr, ns, Kimg, 1, n_ctx, d)) != ZWG_OK) return rc;
         if ((rc = linear_f16_image(ctx, A, rows, ns, w->v_w, w->v_b, ns, Vimg, 2, n_ctx, d)) != ZWG_OK) return rc;
@@ -73,12 +73,12 @@ int zwg_encoder_layer_dev(zwg_ctx *ctx, float *x, uint64_t n_windows, uint64_t n
         bt.out_bstride = n_ctx * ns;
         if ((rc = attention_images_dev(ctx, Q, Kimg, Vimg, tiles, sh, bt, A)) != ZWG_OK) return rc;
     } else { // q | k | v rows of B, read by attention through its strides
-        if ((rc = zwg_linear_epi_dev(ctx, A, rows, ns, w->q_w, ZWG_W_F16, w->q_b, ns, B, 3 * ns, ZWG_EPI_NONE)) != ZWG_OK)
+        if ((rc = linear_f16_keep(ctx, A, rows, ns, w->q_w, w->q_b, ns, B, 3 * ns, ZWG_EPI_NONE)) != ZWG_OK)
             return rc;
-        if ((rc = zwg_linear_epi_dev(ctx, A, rows, ns, w->k_w, ZWG_W_F16, nullptr, ns, B + ns, 3 * ns, ZWG_EPI_NONE)) !=
+        if ((rc = linear_f16_keep(ctx, A, rows, ns, w->k_w, nullptr, ns, B + ns, 3 * ns, ZWG_EPI_NONE)) !=
             ZWG_OK)
             return rc;
-        if ((rc = zwg_linear_epi_dev(ctx, A, rows, ns, w->v_w, ZWG_W_F16, w->v_b, ns, B + 2 * ns, 3 * ns, ZWG_EPI_NONE)) !=
+        if ((rc = linear_f16_keep(ctx, A, rows, ns, w->v_w, w->v_b, ns, B + 2 * ns, 3 * ns, ZWG_EPI_NONE)) !=
             ZWG_OK)
             return rc;
         zwg_attn_shape sh{};
@@ -105,7 +105,7 @@ int zwg_encoder_layer_dev(zwg_ctx *ctx, float *x, uint64_t n_windows, uint64_t n
         return rc;
     // MLP block (src/encoder.zig:172-175)
     if ((rc = zwg_layer_norm_dev(ctx, x, rows, ns, w->mlp_ln_w, w->mlp_ln_b, 1e-5f, A)) != ZWG_OK) return rc;
-    if ((rc = zwg_linear_epi_dev(ctx, A, rows, ns, w->mlp0_w, ZWG_W_F16, w->mlp0_b, 4 * ns, B, 4 * ns, ZWG_EPI_GELU)) !=
+    if ((rc = linear_f16_keep(ctx, A, rows, ns, w->mlp0_w, w->mlp0_b, 4 * ns, B, 4 * ns, ZWG_EPI_GELU)) !=
         ZWG_OK)
         return rc;
     return zwg_linear_epi_dev(ctx, B, rows, 4 * ns, w->mlp1_w, ZWG_W_F16, w->mlp1_b, ns, x, ns, ZWG_EPI_ADD);

@@ -481,7 +481,7 @@ int run_q8_stream(zwg_ctx *ctx, const float *x, uint64_t m, uint64_t k, const in
 }
 
 int run_linear(zwg_ctx *ctx, const float *x, uint64_t m, uint64_t k, const void *w, uint32_t w_type,
-               const float *scales, const float *bias, uint64_t n, float *out, uint64_t ldo = 0, uint32_t epi = 0) {
+               const float *scales, const float *bias, uint64_t n, float *out, uint64_t ldo = 0, uint32_t epi = 0, bool keep = false) {
     if (ldo == 0) ldo = n;
     const std::string msg = check_linear(m, k, w_type, n);
     if (ldo < n || ldo > 0x7fffffffull) return fail(ctx, "output row stride must be >= n");
@@ -512,10 +512,16 @@ int run_linear(zwg_ctx *ctx, const float *x, uint64_t m, uint64_t k, const void 
     a.k = (int32_t)k;
     a.nb = (int32_t)(k / 32);
     a.epi = epi;
+    a.keep = keep;
     return w_type == ZWG_W_Q8 ? run_tiled<zwg_lin::kWQ8>(ctx, a) : run_tiled<zwg_lin::kWF16>(ctx, a);
 }
 
 } // namespace
+
+int zwg_host::linear_f16_keep(zwg_ctx *ctx, const float *x, uint64_t m, uint64_t k, const void *w, const float *bias,
+                              uint64_t n, float *out, uint64_t ldo, uint32_t epi) {
+    return run_linear(ctx, x, m, k, w, ZWG_W_F16, nullptr, bias, n, out, ldo, epi, true);
+}
 
 int zwg_host::linear_f16_image(zwg_ctx *ctx, const float *x, uint64_t rows, uint64_t k, const void *w,
                                const float *bias, uint64_t n, void *img, int kind, uint64_t n_ctx, uint64_t d) {

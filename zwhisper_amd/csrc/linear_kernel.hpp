@@ -69,6 +69,7 @@ struct LinearArgs {
     int64_t ldx, ldw, ldo;
     int32_t m, n, k, nb;
     uint32_t epi; // zwg_ew::kEpi*: store v, gelu(v) or out + v, v = x . w + b
+    int32_t keep; // the next launch reads out: stores that stay cached below 128 MB
     // K split over gridDim.y workgroups when a call has too few tiles to fill the GPU: split s
     // takes k in [s k_split, (s + 1) k_split) (a multiple of BK) and stores its raw sums in
     // part[s][m][n]; a second kernel adds the splits in order, then bias and epilogue
@@ -364,12 +365,13 @@ __device__ __forceinline__ void linear_mfma_body(const LinearArgs &a) {
     float *const dst = (KSPLIT ? a.part + (int64_t)split * a.m * a.n : a.out) + (int64_t)m0 * ldd + n0;
     const int64_t dst_span = (int64_t)(min(BM, a.m - m0) - 1) * ldd + (a.n - n0); // elements from (m0, n0) on
     if (ldd % 4 == 0 && a.n % 4 == 0 && (reinterpret_cast<uintptr_t>(dst) & 15) == 0 && dst_span < 0x1fffffffll) {
-        // A plain or GELU output of 128 MB or more (half the Infinity Cache) goes out non-temporal: its
-        // bursts of 16-byte stores would push out the x rows that the neighbouring column tiles re-read
-        // (24000 x 512 x 2048 with GELU, 197 MB, into alternating buffers: 146 us, 124 non-temporal).  A
-        // smaller one stays cached for the call that reads it next (base.en's layer over 4 windows,
-        // hidden rows of 49 MB: 205 us of the 4-byte kernel's 229, non-temporal 224 of 239).
-        const bool nt = !KSPLIT && (int64_t)a.m * a.n >= (32ll << 20);
+        // Plain and GELU outputs go out non-temporal: bursts of 16-byte stores would push out the x rows that
+        // the neighbouring column tiles re-read (calls by themselves, into alternating buffers: 24000 x 512
+        // x 512 44 us cached, 32 non-temporal; 10000 x 512 x 2048 with GELU 76 and 60, 24000 rows 142 and
+        // 121; base.en's cross keys and values of 32 windows 949 and 912).  An output that the next launch
+        // reads (keep) stays cached while it and its x fit the Infinity Cache (base.en's encoder layer over
+        // 4 windows, hidden rows of 49 MB: 212 us, non-temporal 226; over 16, 197 MB: 666 and 645).
+        const bool nt = !KSPLIT && !(a.keep && (int64_t)a.m * a.n < (32ll << 20));
         const __amdgpu_buffer_rsrc_t o_dst = rsrc(dst, (uint32_t)(dst_span * 4));
         __syncthreads(); // every wave is past its last operand read
         float *const tile = reinterpret_cast<float *>(lds) + wave * kCh * kLd;

@@ -71,6 +71,9 @@ int ensure_stage(zwg_ctx *ctx, int i, uint64_t bytes);
 // the rows are contiguous, else one copy of the whole span into pinned staging and row copies on
 // the host.
 int download_rows(zwg_ctx *ctx, float *dst, const float *src, uint64_t n_rows, uint64_t cols, uint64_t stride);
+// zwg_linear_epi_dev with f16 weights for an output that the next launch reads (LinearArgs keep).
+int linear_f16_keep(zwg_ctx *ctx, const float *x, uint64_t m, uint64_t k, const void *w, const float *bias, uint64_t n,
+                    float *out, uint64_t ldo, uint32_t epi);
 // The encoder layer's K/V path (kv_image.hpp): the f16 linear layer writing K (kind 1) or V
 // (kind 2) tile images in place of f32 rows -- rows = items * n_ctx (n_ctx % 4 == 0), n = heads * d
 // (d 64 or 128) -- and the dense x3 attention reading them (q, out and the shape as for
