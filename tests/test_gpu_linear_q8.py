@@ -371,7 +371,9 @@ def test_two_stage_groups(torch, ctx, m, k, n):
 # multiple of 4 (4-byte stores), of 32 or of a tile; stage counts odd, even and past three.
 PACKED_CASES = [(1, 512, 70), (32, 288, 33), (31, 8960, 130), (33, 768, 257), (64, 8960, 1536), (129, 4864, 897),
                 (200, 1280, 4100), (48, 1376, 16386), (64, 544, 40004), (7, 480, 9001), (256, 96, 8200),
-                (300, 800, 4100), (1100, 3104, 1030)]
+                (300, 800, 4100), (1100, 3104, 1030),
+                # more than 256 rows whose blocks end in an almost empty round: the tiled kernel; and past it
+                (400, 896, 4864), (1300, 896, 4864), (1100, 928, 8200)]
 
 
 @pytest.mark.parametrize("epilogue", ["none", "gelu", "add"])

@@ -656,15 +656,26 @@ int run_q8w_token_step(zwg_ctx *ctx, const float *x, uint64_t m, uint32_t n_w, c
 }
 
 // Calls of more than 256 rows that take the packed kernels (64-row blocks, unsplit) rather than the
-// tiled one: wide outputs, and long k with enough blocks to fill half the chip.  Measured against the
-// tiled kernel (its k split included): x 1536 x 8960 and x 896 x 4864 at 257 to 2048 rows 1.03 to 1.6
-// times as fast; 8960 x 1536 at 512 rows (96 blocks) 0.95, at 700 (132) 1.24; 4864 x 896 at 1001 rows
-// (112) 0.98, at 1500 (168) 1.23; 3072 x 768 at 1500 (144) 1.12; 512 x 2048 0.8 at any size.  The
-// split x needs room in the workspace.
+// tiled one: wide outputs (n >= 4096, k >= 768), and long k with enough 64 x 128 blocks to fill half the
+// chip -- where the blocks' rounds over the 256 CUs, three at a time on each, are fuller than the
+// tiled kernel's.  Swept against it over k 768 .. 2048, n 4096 .. 8960 and 257 .. 2048 rows:
+//   up to 256 blocks   0.70 to 0.99 of its time (896 x 4864 at 384 rows 18.7 us, tiled 20.2)
+//   257 to 384         0.93 to 1.19 at k below 1536 (385 rows 22.6, tiled 22.0), 0.86 to 1.02 from there on
+//   385 to 768         0.74 to 1.09, the longer k the better
+//   769 to 1024        0.92 to 1.23 at every k (a fourth block for some CUs; 1300 rows 41.8, tiled 38.9), but
+//                      0.65 to 0.75 where the tiled call has more than two 128 x 128 tiles per CU
+//   more               0.72 to 0.97
+// Long k: 8960 x 1536 at 640 rows (120 blocks) 1.13, at 700 (132) 0.88; 4864 x 896 at 1100 rows (126) 1.07,
+// at 1300 (147) 0.93; 3072 x 768 from 1300 rows (126) on 0.98 to 1.02.  Narrow outputs of short k: 512 x
+// 2048 at 1001 rows 1.26.  The split x needs room in the workspace.
 bool q8p_takes_rows(const zwg_ctx *ctx, uint64_t m, uint64_t k, uint64_t n) {
     const uint64_t n_chunks = (k + zwg_lin::kQ8Chunk - 1) / zwg_lin::kQ8Chunk, nz = (m + 63) / 64;
     if (nz > 65535 || nz * n_chunks * zwg_lin::q8_chunk_halves<2>() * 2 > ctx->workspace_bytes) return false;
-    return (n >= 4096 && k >= 768) || (k >= 3072 && nz * ((n + 127) / 128) >= 128);
+    const uint64_t blocks = nz * ((n + 127) / 128);
+    if (!(n >= 4096 && k >= 768) && !(k >= 3072 && blocks >= 128)) return false;
+    if (blocks > 256 && blocks <= 384) return k >= 1536;
+    if (blocks > 768 && blocks <= 1024) return tiles(m, n, 128, 128) > 512;
+    return true;
 }
 
 int run_linear_q8w(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *w, const float *bias, float *out,
