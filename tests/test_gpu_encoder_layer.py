@@ -223,7 +223,8 @@ def composed_layer(torch, ctx, xd, n_windows, n_ctx, ns, n_head, wd):
 # (windows, frames, n_state, heads): base.en and tiny.en windows (1500 frames: the last 32-key tile
 # holds 28 keys), head dim 128 with a last tile of 4 keys, whole tiles only, and 70 frames (not a
 # multiple of 4: no images, the f32 path)
-IMAGE_SHAPES = [(2, 1500, 512, 8), (1, 1500, 384, 6), (2, 68, 256, 2), (3, 64, 128, 2), (2, 70, 128, 2)]
+IMAGE_SHAPES = [(2, 1500, 512, 8), (1, 1500, 384, 6), (2, 68, 256, 2), (3, 64, 128, 2), (2, 70, 128, 2),
+                (6, 1500, 384, 6), (9, 1500, 512, 8)]  # 128 x 128 and 64 x 256 projection tiles
 
 
 @pytest.mark.parametrize("n_windows,n_ctx,ns,n_head", IMAGE_SHAPES)

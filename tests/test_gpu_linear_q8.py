@@ -233,6 +233,8 @@ GROUPS = [
     (768, [(768, True), (768, False), (768, True)]),
     # Qwen2.5-1.5B MLP gate and up (src/llm.zig:203-205)
     (1536, [(8960, False), (8960, False)]),
+    # long k: several chunks per workgroup, at 100 rows in 256-column tiles
+    (4864, [(1666, True), (896, False)]),
     # four sets, none a multiple of 128 rows, mixed biases
     (544, [(130, True), (33, False), (257, True), (96, False)]),
 ]
@@ -365,15 +367,19 @@ def test_two_stage_groups(torch, ctx, m, k, n):
     assert np.array_equal(outs[0], outs[1])
 
 
-# One case per branch of the packed kernels' dispatch, at the edges of their tiles: one chunk of k per
-# workgroup (k split, 64-column tiles), several (128 or 256 columns), unsplit calls with fewer and more
-# 128-column units than CUs, calls of more than 256 rows on the packed kernels; one and two m-tiles and 64-row blocks with a ragged last one; n not a
-# multiple of 4 (4-byte stores), of 32 or of a tile; stage counts odd, even and past three.
-PACKED_CASES = [(1, 512, 70), (32, 288, 33), (31, 8960, 130), (33, 768, 257), (64, 8960, 1536), (129, 4864, 897),
-                (200, 1280, 4100), (48, 1376, 16386), (64, 544, 40004), (7, 480, 9001), (256, 96, 8200),
-                (300, 800, 4100), (1100, 3104, 1030),
-                # more than 256 rows whose blocks end in an almost empty round: the tiled kernel; and past it
-                (400, 896, 4864), (1300, 896, 4864), (1100, 928, 8200)]
+# One case or more per branch of the packed kernels' dispatch, at the edges of their tiles: n not a multiple
+# of 4 (4-byte stores), of 32 or of a tile, a ragged last row block, stage counts odd, even and past three.
+PACKED_CASES = [
+    # up to 32 rows: one chunk of k per workgroup (64 columns), several (128 columns; 6 and 8 stages, 2 and 4)
+    (1, 512, 70), (32, 288, 33), (31, 8960, 130), (32, 8960, 1536), (17, 4864, 1537),
+    # unsplit, fewer 64-column units than CUs (two waves per SIMD on halves of each stage) and more
+    (7, 480, 9001), (32, 800, 33000),
+    # 64-row blocks, k split: one chunk per workgroup, several in 128-column and in 256-column tiles
+    (33, 768, 257), (64, 8960, 1536), (129, 4864, 897), (256, 4864, 896), (250, 4864, 1666),
+    # unsplit, fewer 128-column units than CUs and more, x split in the kernel and by a pass of its own
+    (200, 1280, 4100), (48, 1376, 16386), (64, 544, 40004), (256, 96, 8200),
+    # more than 256 rows: both of those, and the tiled kernel where the blocks end in an almost empty round
+    (300, 800, 4100), (1100, 3104, 1030), (1100, 928, 8200), (400, 896, 4864), (1300, 896, 4864)]
 
 
 @pytest.mark.parametrize("epilogue", ["none", "gelu", "add"])

@@ -388,6 +388,35 @@ def test_forward_bit_exact_with_composed_calls(torch, ctx, ne, H, Hk, nff):
             pos += n
 
 
+@pytest.mark.parametrize("ne,H,Hk,nff,batches", [(896, 14, 2, 4864, (256, 33)), (1536, 12, 2, 8960, (24,))],
+                         ids=["rows256", "rows24"])
+def test_forward_bit_exact_long_down_projections(torch, ctx, ne, H, Hk, nff, batches):
+    """Down projections of many chunks of k: 256 rows take 256-column tiles, 24 rows several chunks per
+    workgroup; their sums add into x and normalise it.  As the separate calls, bit for bit."""
+    import zwhisper_amd as z
+    from zwhisper_amd import _lib
+
+    rng = np.random.default_rng(nff)
+    n_layer, n_vocab, n_ctx = 2 if ne < 1000 else 1, 300, 304
+    mdl = model(rng, ne, H, Hk, nff, n_layer, n_vocab)
+    with contextlib.ExitStack() as st:
+        lm = st.enter_context(make_llm(z, ctx, mdl, H, Hk, nff, n_ctx, 1))
+        kv = st.enter_context(z.KVCache(ctx, n_layer, 1, n_ctx, Hk, ne // H, _lib.KV_KT, 1e6))
+        la, lb = torch.empty(n_vocab, device="cuda"), torch.empty(n_vocab, device="cuda")
+        pos = 0
+        for n in batches:
+            print(f"forward batch of {n} at {pos}, n_embd={ne} n_ff={nff}", flush=True)
+            toks = rng.integers(0, n_vocab, n).astype(np.int32)
+            lm.forward(torch.from_numpy(toks).cuda(), pos, la, 0)
+            composed_forward(torch, ctx, lm, kv, mdl["embd"], H, Hk, toks, pos, 0, lb)
+            torch.cuda.synchronize()
+            assert bool(torch.isfinite(la).all()) and torch.equal(la, lb), n
+            for li in range(n_layer):
+                a, b = lm.kv.read(li, 0), kv.read(li, 0)
+                assert np.array_equal(a[0], b[0]) and np.array_equal(a[1], b[1]), (n, li)
+            pos += n
+
+
 def test_forward_matches_steps(torch, ctx):
     """A prompt batch through zwg_llm_forward_dev and the same tokens one by one through
     zwg_llm_step_dev (other kernels): the last token's logits and the caches within f32
