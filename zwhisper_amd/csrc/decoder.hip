@@ -7,16 +7,16 @@
 //
 //   X = te.row(tok) + pe[pos]; A = attn_ln(X)        q8p_embed_ln_kernel (one launch)
 //   per layer:
-//     Q = q(A); k(A), v(A) -> self cache rows at pos  stream + linear_split_sum_qkv_kernel, which
+//     Q = q(A); k(A), v(A) -> self cache rows at pos  int8 + linear_split_sum_qkv_kernel, which
 //                                                     also writes the key counts pos + 1
 //     T = attention(Q, self cache[0 .. pos])           decode kernel (+ merge)
-//     X += o(T); A = cross_ln(X)                       stream + linear_split_sum_add_ln_wide_kernel
-//     T = attention(cq(A), cross cache)                stream (partials to P) + decode kernel, whose
+//     X += o(T); A = cross_ln(X)                       int8 + linear_split_sum_add_ln_wide_kernel
+//     T = attention(cq(A), cross cache)                int8 (partials to P) + decode kernel, whose
 //                                                     q load adds the partials and bias (+ merge)
-//     X += co(T); A = mlp_ln(X)                        stream + linear_split_sum_add_ln_wide_kernel
-//     H = gelu(mlp0(A))                                stream + split sum (GELU in its store)
+//     X += co(T); A = mlp_ln(X)                        int8 + linear_split_sum_add_ln_wide_kernel
+//     H = gelu(mlp0(A))                                int8 + split sum (GELU in its store)
 //     X += mlp1(H); A = next layer's attn_ln(X), or the final ln after the last layer
-//   logits = A . te^T                                  stream (unsplit)
+//   logits = A . te^T                                  int8 (unsplit)
 //
 // 12-14 launches per layer where the same step as separate calls (layer norm, q/k/v projections,
 // append, add) takes 19-21.  The fused launches form the same values in the same order as the

@@ -135,17 +135,15 @@ std::string check_linear(uint64_t m, uint64_t k, uint32_t w_type, uint64_t n) {
     return "";
 }
 
-// Q8 with m <= 64: x split into hi/lo halves by linear_q8_xprep_kernel into the workspace, then
-// the weight-streaming kernel.  Four waves of S slabs of 32 weight rows per workgroup (S = 2 when
-// that alone makes >= 256 workgroups, else 1); a call of fewer than 512 workgroups splits k over
-// more, at chunk granularity, up to about ZWG_Q8P_SPLIT_TARGET of them, as long as the partial
-// sums fit the workspace.  (Raw-layout weights; the resident packed ones go through run_q8p_group.)
+// Raw-layout Q8 weights (the resident packed ones go through run_q8p_group) with m <= 64: x split into
+// hi/lo halves by linear_q8_xprep_kernel into the workspace, then the weight-streaming kernel.  Four
+// waves of S slabs of 32 weight rows per workgroup (S = 2 when that alone makes >= 256 workgroups, else
+// 1); a call of fewer than 512 workgroups splits k over more, at chunk granularity, up to about
+// ZWG_Q8P_SPLIT_TARGET of them, as long as the partial sums fit the workspace.
 //
-// Workgroups a split call is split up to (within its k chunks).  Only the Qwen2.5-1.5B down
-// projection (k = 8960: 18-way at 256, 35-way at 512) reaches it; its projections alone measured
-// 2163 / 2048 / 1960 / 1964 / 1963 us at 128 / 192 / 256 / 512 / 1024, and its whole token step,
-// whose down projection's sums add into x and normalise it in one row kernel, 4.117 / 4.073 /
-// 4.074 ms at 512 / 384 / 256 (paired runs): that kernel reads half the partials at 256
+// Units that a split call is split up to (within its k chunks), both layouts alike.  Packed calls, at
+// 128 / 256 / 512: two layers of Qwen2.5-1.5B's token step over 64 sequences 303 / 297 / 307 us, over 32
+// 274 / 264 / 261, small.en's decoder step over 32 windows 1493 / 1461 / 1444, over one 876 / 832 / 833
 #ifndef ZWG_Q8P_SPLIT_TARGET
 #define ZWG_Q8P_SPLIT_TARGET 256
 #endif
@@ -191,24 +189,24 @@ int run_q8_stream_mt(zwg_ctx *ctx, const zwg_lin::Q8Args &base) {
 // preceded by one x split for the 64-row calls that do not split x themselves, and when k is split,
 // one split sum over every set's outputs.  The k split is chosen from the group's total count of
 // units of q8p_unit<MT>() weight rows, as for a single call; the kernel and its tile are chosen
-// below from the split and the unit count, and do not change the sums.
+// below from the split and the unit count.  The tiles give the same sums, except that the unsplit
+// forms with two waves on halves of each stage (fewer than 256 units) add two halves' sums at the end.
 template <int MT>
 constexpr int q8p_unit() { return MT == 1 ? 64 : 128; }
-// k is split only for calls below this many workgroups.  A call at or above it streams unsplit:
-// its partial sums would be as large as half its weights (the Qwen2.5-1.5B gate/up, 140
-// workgroups: split 3 ways, 13.8 MB of partials for 27.5 MB of weights).  Measured on one box,
-// splitting below 512 / 160 / 100 / 64 workgroups: Qwen2.5-1.5B decode step 2297 / 2297 / 2126 /
-// 2118 us, small.en decoder step 690 / 675 / 675 / 675 us.
+// k is split only for calls below this many units.  A call at or above it runs unsplit: its partial
+// sums would be as large as half its weights (the Qwen2.5-1.5B gate/up, 140 units: split 3 ways, 13.8 MB
+// of partials for 27.5 MB of weights).  Splitting below 64 / 128 / 256: two layers of Qwen2.5-1.5B's token
+// step over 64 sequences 298 / 297 / 310 us, of 0.5B's 201 / 208 / 210, small.en's decoder step over 32
+// windows 1461 / 1461 / 1463, 100 rows of a Qwen2.5-0.5B prompt 1645 / 1647 / 1831
 #ifndef ZWG_Q8P_SPLIT_BELOW
 #define ZWG_Q8P_SPLIT_BELOW 128
 #endif
-// calls of up to this many rows stream the resident weights (64-row blocks of one launch); more
-// rows take the tiled GEMM
+// Calls of up to this many rows take the packed kernels whatever their shape, k split where that
+// helps, and split x themselves when their row blocks are several; the fused calls (q/k/v into the cache,
+// residual + norm, SwiGLU) take as many.  Longer ones take them unsplit where q8p_takes_rows says so.
 #ifndef ZWG_Q8P_STREAM_ROWS
 #define ZWG_Q8P_STREAM_ROWS 256
 #endif
-#define ZWG_Q8P_FUSED_ROWS 256
-
 
 // Row kernels of n <= 4096 floats (a wave per row, n / 256 float4 per lane, rounded up, or a thread per
 // float4), one row per workgroup: a decode step's few rows then read their partials through as many CUs as
@@ -263,9 +261,8 @@ struct Q8PartsOut {
     int max_parts;
     int n_split;
 };
-// calls of several 64-row blocks (gridDim.z) take their own split rule: split below the same
-// count, up to about 256 workgroups (the Qwen2.5-0.5B prompt's 256-row calls, per 2048-token
-// prompt: 22.43 ms at 512, 22.19 at 256; splitting calls of up to 512 or 1024 workgroups: 23.9 ms)
+// calls of several 64-row blocks (gridDim.z) take their own split target: the Qwen2.5-0.5B prompt's
+// 256-row batch 2083 / 2052 / 2182 us at 128 / 256 / 512, 100 rows 1645 us at each
 #ifndef ZWG_Q8P_SPLIT_BELOW_Z
 #define ZWG_Q8P_SPLIT_BELOW_Z ZWG_Q8P_SPLIT_BELOW
 #endif
@@ -343,8 +340,10 @@ hipError_t launch_q8p(const zwg_lin::Q8Args &a, const zwg_lin::Q8Group &g, const
         return launch_q8p_tile<false, 1, 4, 1, 4>(a, g, xcvt, XS, n_split, nz, st);
     } else {
         // one chunk per workgroup: 64 columns on four waves (64 x 1536 x 1536 in 6 splits 5.7, 128
-        // columns 6.6, the long kernel 6.9) while those are at most one per CU (65 x 896 x 4864 in 4 splits,
-        // 608 of them, one at a time per CU: 19.6 with the split sum, the long kernel 14.5)
+        // columns 6.6, the long kernel 6.9) while those are at most one per CU.  Two fit a CU: up to 512
+        // calls by themselves gain (with the split sum, 160 x 1536 x 1536, 432 of them, 13.8 -> 11.9), but rows
+        // that arrive split lose (the Qwen2.5-0.5B prompt's 256-row batch, whose q/k/v are 288 of them, 2137
+        // -> 2145); past 512 all do (129 x 1536 x 2048, 576, 13.4 -> 15.7)
         if (n_split > 1 && a.chunks_per_split == 1 && 2 * units * n_split <= 256) return launch_q8p_tile<true, 2, 2, 2, 4>(a, g, xcvt, XS, n_split, nz, st);
         // more units than CUs, split: 256 columns (256 x 4864 x 896 in 10 splits 14.5, 128 columns
         // 16.1); fewer: 128 columns (64 x 8960 x 1536 in 18 splits 12.0, 256 columns 13.9)
@@ -384,11 +383,11 @@ int run_q8p_group(zwg_ctx *ctx, const zwg_lin::Q8Args &base, zwg_lin::Q8Group g,
     const int nz = (int)((m + 32 * MT - 1) / (32 * MT));
     if (nz > 1 && (MT != 2 || po)) return fail(ctx, "the partials call takes at most 64 rows");
     const int64_t gxz = gx * nz;
-    const bool split_k = q8p_split_k(gxz, n_chunks, nz) && m <= ZWG_Q8P_FUSED_ROWS;
+    const bool split_k = q8p_split_k(gxz, n_chunks, nz) && m <= ZWG_Q8P_STREAM_ROWS;
     // xcvt_in (64-row blocks): x was split by the caller's previous launch.  The partial sums keep
     // the place (and so the split count) the call has without it.  Calls of at most 256 rows whose
     // row blocks share one launch split x themselves; longer ones (always unsplit) take the pass.
-    const bool long_m = m > ZWG_Q8P_FUSED_ROWS;
+    const bool long_m = m > ZWG_Q8P_STREAM_ROWS;
     const bool xs_own = q8p_splits_x_itself<MT>(gxz, n_chunks) || (nz > 1 && !long_m);
     const bool XS = xs_own && !(MT == 2 && xcvt_in);
     if (resln && resln->xcvt && MT != 2) return fail(ctx, "split rows for the next call come from calls of more than 32 rows");
@@ -426,7 +425,7 @@ int run_q8p_group(zwg_ctx *ctx, const zwg_lin::Q8Args &base, zwg_lin::Q8Group g,
         if (e != hipSuccess) return fail_hip(ctx, "linear (int8) x preparation launch", e);
     }
     e = launch_q8p<MT>(a, g, xcvt, XS, gxz, n_split, nz, ctx->stream);
-    if (e != hipSuccess) return fail_hip(ctx, "linear (int8 stream) kernel launch", e);
+    if (e != hipSuccess) return fail_hip(ctx, "linear (packed int8) kernel launch", e);
     if (kvs) {
         const int64_t threads = (int64_t)m * (kvs->n_head + 2 * kvs->n_head_kv) * (kvs->d / 8);
         const int bs = small_block(threads);
@@ -626,8 +625,7 @@ void detach_q8w(void *obj) {
     w->ctx = nullptr;
 }
 
-// The token-step path (m <= 64) over n_w resident weight sets sharing x and k (checked by the
-// callers).
+// The packed kernels over n_w resident weight sets sharing x and k (checked by the callers).
 int run_q8w_token_step(zwg_ctx *ctx, const float *x, uint64_t m, uint32_t n_w, const zwg_q8w *const *w,
                        const float *const *bias, float *const *out, uint32_t epi,
                        const zwg_lin::Q8KvStore *kvs = nullptr, const zwg_lin::Q8ResLn *resln = nullptr,
@@ -762,7 +760,7 @@ int zwg_host::linear_q8w_qkv_kv(zwg_ctx *ctx, const float *x, uint64_t m, const 
 }
 
 // x += xin . W^T + bias and ln_out = the norm of x (layer norm with ln_w, ln_b, or RMS norm with
-// ln_w; eps) for a decode step's or a prompt batch's rows (m <= 256, n <= 4096): one stream launch and
+// ln_w; eps) for a decode step's or a prompt batch's rows (m <= 256, n <= 4096): one packed launch and
 // linear_split_sum_add_ln_wide_kernel; a call too short to split k (k <= 256) runs the add epilogue and
 // the norm as two launches, with the same results.  xcvt_out (more than 32 rows): ln_out also split
 // for the next call (q8w_xcvt_halves(m, n) halves), which takes it as xcvt_in.
@@ -796,7 +794,7 @@ int zwg_host::linear_q8w_add_ln(zwg_ctx *ctx, const float *xin, uint64_t m, cons
 uint64_t zwg_host::q8w_stream_rows() { return ZWG_Q8P_STREAM_ROWS; }
 
 // out = silu(x . gate^T) * (x . up^T) for at most q8w_stream_rows() rows (src/llm.zig:207-210):
-// one stream launch over both weight sets (a SwiGLU pair), plus one SwiGLU split sum when k is
+// one packed launch over both weight sets (a SwiGLU pair), plus one SwiGLU split sum when k is
 // split; the same values as the two projections' group call followed by the SiLU-mul kernel.
 // xcvt_in as for linear_q8w_group_xcvt.
 int zwg_host::linear_q8w_swiglu(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *gate, const zwg_q8w *up,
@@ -823,8 +821,7 @@ uint64_t zwg_host::q8w_xcvt_halves(uint64_t m, uint64_t k) {
 }
 
 // A grouped token-step call (as zwg_linear_q8w_group_dev, m <= 64) whose x was split by the
-// previous call (linear_q8w_add_ln's xcvt_out, from the same rows); used where the call streams
-// its x from a split pass (33..64 rows, unsplit k), ignored where it splits x itself.
+// previous call (linear_q8w_add_ln's xcvt_out, from the same rows; 33..64 rows), or xcvt_in nullptr.
 int zwg_host::linear_q8w_group_xcvt(zwg_ctx *ctx, const float *x, uint64_t m, uint32_t n_w, const zwg_q8w *const *w,
                                     const float *const *bias, float *const *out, const _Float16 *xcvt_in) {
     if (n_w == 0 || n_w > (uint32_t)zwg_lin::kQ8MaxGroup || !w || !out) return fail(ctx, "n_w must be 1..4");

@@ -11,24 +11,30 @@
 // block's two MFMAs per term accumulate hi*q and lo*q in f32, and the block sum is scaled in f32
 // on the VALU.  |x| must stay within f16's range (65504).
 //
-// Two kernels:
+// Three families of kernels (linear.hip chooses):
 //
-// * linear_q8_stream_kernel<MT, S>: m <= 64 (decoder and LLM token steps, logits).  The weights
-//   are the stream: every int8 byte is read from HBM once, 16 bytes per lane per load (one Q8
+// * linear_q8p_short_kernel, linear_q8p_long_kernel: resident weights in the packed layout (Q8Packed),
+//   token steps, logits, prompt batches of up to 256 rows and the longer calls that they win.  32- or
+//   64-row blocks; each stage of x sits in LDS split into hi/lo halves in the MFMA A-operand order, and
+//   every wave streams its own slabs of 32 weight rows into registers.
+//
+// * linear_q8_stream_kernel<MT, S>: weights as the caller has them (int8 [n][k]), m <= 64.  The
+//   weights are the stream: every int8 byte is read from HBM once, 16 bytes per lane per load (one Q8
 //   block of 32 weight rows per wave-load).  A workgroup of 4 waves owns 4*S slabs of 32 weight
 //   rows and walks k in chunks of 256 (8 blocks).  x is split into hi/lo halves once per call by
 //   linear_q8_xprep_kernel, in the exact order the MFMA A operand wants it; each workgroup copies
 //   a chunk of it into LDS with direct global-to-LDS loads (no VGPRs, no VALU), issued before the
 //   chunk's weight loads so the wait for x never waits on the weights.  An operand read is then
 //   1 KB contiguous per wave (conflict-free ds_read_b128).
-//   v_mfma_f32_32x32x16_f16 with A = x rows, B = weight rows: lane l's 16 weight bytes
-//   q[row l%32][kb + 16 (l/32) .. +16] feed the block's two k-steps (bytes 0-7, then 8-15), and
-//   the result column l%32 is the weight row, so the block's scale is one f32 per lane.
-//   When the weight rows alone give too few workgroups to fill the chip, k is split over
-//   gridDim.y and linear_split_sum_kernel adds the partial sums in a fixed order.
 //
-// * linear_mfma_kernel<BM, BN, true> (linear_kernel.hpp): larger m, the tiled GEMM with the
-//   weight tile widened to f16 on its way into LDS and the same per-block scaling.
+// * linear_mfma_kernel<BM, BN, kWQ8 or kWQ8P> (linear_kernel.hpp): the remaining calls of more rows, the
+//   tiled GEMM with the weight tile widened to f16 on its way into LDS and the same per-block scaling.
+//
+// The first two use v_mfma_f32_32x32x16_f16 with A = x rows, B = weight rows: lane l's 16 weight bytes
+// q[row l%32][kb + 16 (l/32) .. +16] feed the block's two k-steps (bytes 0-7, then 8-15), and
+// the result column l%32 is the weight row, so the block's scale is one f32 per lane.  When the
+// weight rows alone give too few workgroups to fill the chip, k is split over gridDim.y and a
+// split-sum kernel adds the partial sums in a fixed order.
 //
 // MFMA operand layout (v_mfma_f32_32x32x16_f16, measured on the device): lane l, half s of A is
 // A[l % 32][8 (l / 32) + s], of B is B[8 (l / 32) + s][l % 32]; result register r of lane l is
@@ -46,11 +52,11 @@
 namespace zwg_lin {
 
 constexpr int kQ8Block = 32;                // src/gemm.zig:194
-constexpr int kQ8Chunk = 256;               // k per LDS chunk of the stream kernel
+constexpr int kQ8Chunk = 256;               // k per chunk: of the packed layout, the split x and the stream kernel's LDS
 constexpr int kQ8ChunkBlocks = kQ8Chunk / kQ8Block;
 constexpr int kQ8Threads = 256;
-// The packed weights and scales are read once per call: non-temporal loads (cache policy nt)
-// stream them past the caches, which keep the x stages every workgroup reuses.
+// Cache policy nt: packed weights that one row block reads once stream past the caches, which keep the
+// x stages that every workgroup reuses (Q8pTile::POLICY).
 constexpr int kQ8CachePolicyNT = 2;
 
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));

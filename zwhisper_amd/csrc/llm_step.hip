@@ -8,18 +8,18 @@
 //   X = embd.row(tok); H = rmsNorm(X, attn_norm)      q8p_embed_ln_kernel (RMS), one launch
 //   per layer:
 //     Q = rope(q(H)); rope(k(H)) -> K^T cache, v(H) -> V cache at pos
-//                                                    stream + linear_split_sum_qkv_kernel, which
+//                                                    int8 + linear_split_sum_qkv_kernel, which
 //                                                    also writes the key counts pos + 1
 //     T = attention(Q, caches[0 .. pos])             decode kernel over transposed keys (+ merge)
-//     X += o(T); H = rmsNorm(X, ffn_norm)            stream + linear_split_sum_add_ln_wide_kernel
+//     X += o(T); H = rmsNorm(X, ffn_norm)            int8 + linear_split_sum_add_ln_wide_kernel
 //                                                    (RMS), which also splits H into f16 hi/lo
 //                                                    halves for the next call (more than 32 rows)
-//     G = silu(gate(H)) * up(H)                      one stream launch over both weight sets, each
+//     G = silu(gate(H)) * up(H)                      one launch over both weight sets, each
 //                                                    workgroup on the same columns of both (a
 //                                                    SwiGLU pair; + one split sum when k is split);
 //                                                    G written split for the down projection
 //     X += down(G); H = next layer's attn_norm(X), or the output norm after the last layer
-//                                                    stream + the sum, residual add and norm
+//                                                    int8 + the sum, residual add and norm
 //   logits = H . output^T                           one launch (33..64 sequences: x split by the
 //                                                    last down projection's sum kernel)
 //
@@ -237,7 +237,7 @@ int zwg_llm_forward_dev(zwg_ctx *ctx, const zwg_llm *lm, const int32_t *tokens, 
     sh.out_stride = ne;
     sh.kt_stride = kv->desc.n_ctx;
     sh.causal = 1;
-    // batches the int8 calls stream (at most q8w_stream_rows() rows) take the fused launches of the
+    // batches of at most q8w_stream_rows() rows take the fused launches of the
     // decode step: the q/k/v projections writing the cache, and the residual projections' split
     // sums adding into x and normalising it for the next block, with the same results
     const bool fused = n <= q8w_stream_rows();

@@ -98,9 +98,9 @@ int linear_q8w_parts(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *w,
 int linear_q8w_qkv_kv(zwg_ctx *ctx, const float *x, uint64_t m, const zwg_q8w *const *w, const float *const *bias,
                       float *q_out, zwg_kv *kv, uint64_t layer, uint64_t seq0, const int32_t *pos_dev,
                       int32_t *n_kv_out, int64_t pos0 = -1, const _Float16 *xcvt_in = nullptr);
-// rows up to which the int8 calls stream the resident weights (and the fused calls take)
+// rows up to which every int8 call takes the packed kernels (and the fused calls take)
 uint64_t q8w_stream_rows();
-// out = silu(x . gate^T) * (x . up^T), m <= q8w_stream_rows() (one stream launch over both sets);
+// out = silu(x . gate^T) * (x . up^T), m <= q8w_stream_rows() (one launch over both sets);
 // xcvt_in (more than 32 rows): x as linear_q8w_add_ln split it; xcvt_out (likewise, n % 128 == 0): the
 // output goes there split for the next call (q8w_xcvt_halves(m, n) halves; rows past m unwritten) and
 // not to out
