@@ -134,12 +134,12 @@ def kernel_notes(objects):
 
 def test_kernels_do_not_spill(objects):
     """No kernel spills a vector register.  The split sum + residual + norm kernel (a thread per float4 column,
-    up to 1024 of them) keeps four waves per SIMD at every row width: 128 registers."""
+    up to 1024 of them) keeps three waves per SIMD for rows of up to 2048 floats and four for wider ones."""
     kernels, rows = 0, 0
     for name, values in kernel_notes(objects):
         kernels += 1
         assert values["vgpr_spill_count"] == 0, name
         if "linear_split_sum_add_ln_wide" in name:
             rows += 1
-            assert values["vgpr_count"] <= 128, name
+            assert values["vgpr_count"] <= (168 if values["max_flat_workgroup_size"] <= 512 else 128), name
     assert kernels > 100 and rows >= 24  # two norms, twelve row widths

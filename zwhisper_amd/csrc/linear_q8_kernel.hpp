@@ -1108,7 +1108,8 @@ __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(co
     typedef float f4 __attribute__((ext_vector_type(4)));
     constexpr int B = 24;
     constexpr bool kLayerNorm = NORM != zwg_ew::kNormRms;
-    __shared__ f4 rowbuf[64 * R], wbuf[64 * R], bbuf[kLayerNorm ? 64 * R : 1];
+    constexpr bool kPass = R * (kLayerNorm ? 2 : 1) > 8; // the norm's weights through LDS, below
+    __shared__ f4 rowbuf[64 * R], wbuf[kPass ? 64 * R : 1], bbuf[kPass && kLayerNorm ? 64 * R : 1];
     const int c = threadIdx.x; // this thread's float4 column
     const int row = (int)blockIdx.x;
     if (row >= m) return;
@@ -1122,14 +1123,19 @@ __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(co
         xo = xr[c];
         if (bias) bo = reinterpret_cast<const f4 *>(bias)[c];
     }
-    // the norm's weights, each thread its column's, in flight with the partials rather than a round trip
-    // behind them (the small.en decoder step 1460 -> 1436 us over its 36 launches), and to the first wave
-    // through LDS: held in its registers they cost every wave as many, and spilled from R = 14 on (a step
-    // of eight layers of 4096 floats, 64 rows: 961 us so, 771 through LDS)
-    f4 nw = {0.f, 0.f, 0.f, 0.f}, nb = {0.f, 0.f, 0.f, 0.f};
-    if (live) {
-        nw = reinterpret_cast<const f4 *>(r.ln_w)[c];
-        if constexpr (kLayerNorm) nb = reinterpret_cast<const f4 *>(r.ln_b)[c];
+    // the norm's weights for the first wave, in flight with the partials rather than a round trip behind
+    // them (the small.en decoder step 1460 -> 1436 us over its 36 launches).  Up to eight float4s go
+    // straight to its registers (which every wave then has, at no loss: these rows are few workgroups);
+    // of wider rows each thread loads its column's and passes them on through LDS, as in registers they
+    // took a wave per SIMD and spilled from R = 14 on (a step of eight layers of 4096 floats, 64 rows:
+    // 961 us so, 771 through LDS; the Qwen2.5-0.5B prompt's batch, R = 4, 2140 through LDS, 2134 so)
+    f4 nw[kPass ? 1 : R], nb[kPass || !kLayerNorm ? 1 : R];
+#pragma unroll
+    for (int i = 0; i < (kPass ? 1 : R); ++i) {
+        const int at = kPass ? c : c + 64 * i;
+        if (at >= n4 || (!kPass && c >= 64)) continue;
+        nw[i] = reinterpret_cast<const f4 *>(r.ln_w)[at];
+        if constexpr (kLayerNorm) nb[i] = reinterpret_cast<const f4 *>(r.ln_b)[at];
     }
     f4 s = {0.f, 0.f, 0.f, 0.f};
     for (int q0 = 0; q0 < n_split; q0 += B) {
@@ -1149,8 +1155,10 @@ __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(co
         xr[c] = nx;
     }
     rowbuf[c] = nx;
-    wbuf[c] = nw;
-    if constexpr (kLayerNorm) bbuf[c] = nb;
+    if constexpr (kPass) {
+        wbuf[c] = nw[0];
+        if constexpr (kLayerNorm) bbuf[c] = nb[0];
+    }
     __syncthreads();
     if (c < 64) {
         zwg_ew::ew_f32x4 v[R];
@@ -1159,9 +1167,10 @@ __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(co
         // with xcvt the normalised row also goes back into rowbuf (past n4 it stays zero)
         float *const orow = r.ln_out + (int64_t)row * n;
         f4 *const copy = r.xcvt ? rowbuf : nullptr;
-        const auto w = [&](int i) { return wbuf[c + 64 * i]; };
+        const auto w = [&](int i) { return kPass ? wbuf[c + 64 * i] : nw[kPass ? 0 : i]; };
         if constexpr (kLayerNorm)
-            zwg_ew::layer_norm_with<R>(v, c, n4, w, [&](int i) { return bbuf[c + 64 * i]; }, r.eps, orow, copy);
+            zwg_ew::layer_norm_with<R>(
+                v, c, n4, w, [&](int i) { return kPass ? bbuf[c + 64 * i] : nb[kPass ? 0 : i]; }, r.eps, orow, copy);
         else
             zwg_ew::rms_norm_with<R>(v, c, n4, w, r.eps, orow, copy);
     }
