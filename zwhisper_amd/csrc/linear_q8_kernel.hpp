@@ -1127,8 +1127,9 @@ __global__ __launch_bounds__(64 * R) void linear_split_sum_add_ln_wide_kernel(co
     // them (the small.en decoder step 1460 -> 1436 us over its 36 launches).  Up to eight float4s go
     // straight to its registers (which every wave then has, at no loss: these rows are few workgroups);
     // of wider rows each thread loads its column's and passes them on through LDS, as in registers they
-    // took a wave per SIMD and spilled from R = 14 on (a step of eight layers of 4096 floats, 64 rows:
-    // 961 us so, 771 through LDS; the Qwen2.5-0.5B prompt's batch, R = 4, 2140 through LDS, 2134 so)
+    // took a wave per SIMD and spilled (layer norm from R = 10, RMS from 14: a step of eight layers of 4096
+    // floats, 64 rows, 961 us so, 771 through LDS; the Qwen2.5-0.5B prompt's batch, R = 4, 2140 through
+    // LDS, 2134 so)
     f4 nw[kPass ? 1 : R], nb[kPass || !kLayerNorm ? 1 : R];
 #pragma unroll
     for (int i = 0; i < (kPass ? 1 : R); ++i) {
