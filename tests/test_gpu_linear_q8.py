@@ -245,7 +245,7 @@ GROUPS = [
 def test_resident_group(torch, ctx, m, gi):
     """zwg_linear_q8w_group_dev: each output against its single call (to f32 rounding: the group's
     k split can differ from a single call's), against f64, and the same call twice bit for bit;
-    m = 100 takes two 64-row blocks of the stream kernel in one launch."""
+    m = 100 takes two 64-row blocks in one launch."""
     import contextlib
 
     k, sets = GROUPS[gi]
@@ -342,7 +342,7 @@ def test_split_calls_in_graph_replays(torch, ctx):
 
 # Unsplit calls of 128-255 workgroups (resident weights): each workgroup's waves form two groups,
 # each over half of the stages of 128 k, summed through LDS.  Shapes: the Qwen2.5-1.5B MLP gate
-# (m = 64 and 33, two m-tiles), a 32-row call (one m-tile, x split in the stream kernel), and k
+# (m = 64 and 33, two m-tiles), a 32-row call (one m-tile, x split in the kernel), and k
 # whose stage count is odd or leaves the second group one stage (k = 416: 4 stages, the last
 # partial; k = 384: 3 stages; k = 288: 3 stages, the last a quarter).
 TWO_GROUP_CASES = [(64, 1536, 17920), (33, 416, 16400), (32, 384, 9000), (17, 8960, 9000), (1, 288, 12000)]

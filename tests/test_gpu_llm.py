@@ -293,7 +293,7 @@ def _ora_model(z, mdl, H, Hk, n_ctx, d, base=1e6):
 
 @pytest.mark.parametrize("ne,H,Hk,nff", [(384, 6, 2, 1024), (512, 4, 2, 1376)], ids=["d64", "d128"])
 def test_forward_against_oracle(torch, ctx, ne, H, Hk, nff):
-    """zwg_llm_forward_dev over prompt batches of 40, 70 (the tiled GEMMs past 64 rows) and 5
+    """zwg_llm_forward_dev over prompt batches of 40, 70 (two 64-row blocks) and 5
     tokens of sequence 1 against Oracle.llm_forward over the same batches: the last token's
     logits within 2e-5 of the largest |logit|, the cache rows within 2e-5 relative."""
     import oracle
@@ -359,7 +359,7 @@ def composed_forward(torch, ctx, lm, kv, embd, H, Hk, toks, pos0, seq, logits):
 @pytest.mark.parametrize("ne,H,Hk,nff", [(384, 6, 2, 1024), (480, 15, 5, 864), (384, 6, 2, 8192)],
                          ids=["d64", "d32", "ff8192"])
 def test_forward_bit_exact_with_composed_calls(torch, ctx, ne, H, Hk, nff):
-    """Prompt batches of at most 256 tokens (40, then 100: two 64-row blocks of the stream kernel,
+    """Prompt batches of at most 256 tokens (40, then 100: two 64-row blocks,
     then 5) through the fused launches (the q/k/v projections writing the cache, the split sums
     adding into x and normalising it) equal the batch as separate calls bit for bit: the logits
     and the cache."""

@@ -231,7 +231,7 @@ class Context:
 
     def linear_q8w_group_dev(self, x, m: int, ws, biases, outs) -> None:
         """outs[j][m][ws[j].n] = x[m][k] . ws[j]^T (+ biases[j]) for up to four resident weight sets
-        sharing k, in one x split, stream launch and split sum (zwg_linear_q8w_group_dev)."""
+        sharing k, in one x split, product launch and split sum (zwg_linear_q8w_group_dev)."""
         n_w = len(ws)
         if not 1 <= n_w <= 4 or len(outs) != n_w or (biases is not None and len(biases) != n_w):
             raise ZwgError("one to four weight sets, with as many outputs (and biases)")
