@@ -340,11 +340,10 @@ def test_split_calls_in_graph_replays(torch, ctx):
             torch.cuda.synchronize()
 
 
-# Unsplit calls of 128-255 workgroups (resident weights): each workgroup's waves form two groups,
-# each over half of the stages of 128 k, summed through LDS.  Shapes: the Qwen2.5-1.5B MLP gate
-# (m = 64 and 33, two m-tiles), a 32-row call (one m-tile, x split in the kernel), and k
-# whose stage count is odd or leaves the second group one stage (k = 416: 4 stages, the last
-# partial; k = 384: 3 stages; k = 288: 3 stages, the last a quarter).
+# Unsplit calls of 128-255 units (resident weights): two waves per slab, each over half of every stage of
+# 128 k, their sums added through LDS.  Shapes: the Qwen2.5-1.5B MLP gate (m = 64 and 33, two m-tiles), a
+# 32-row call (one m-tile, x split in the kernel), and k whose stage count is odd or whose last stage is
+# partial (k = 416: 4 stages, the last partial; k = 384: 3 stages; k = 288: 3 stages, the last a quarter).
 TWO_GROUP_CASES = [(64, 1536, 17920), (33, 416, 16400), (32, 384, 9000), (17, 8960, 9000), (1, 288, 12000)]
 
 
